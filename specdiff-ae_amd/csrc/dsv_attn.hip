@@ -134,6 +134,17 @@ __device__ __forceinline__ bool tmask_keep(const AttnArgs& a, int b, int i, int 
   }
 }
 
+// LDS words of the byte-mask variant's keep-bit window (80 KiB beside the
+// ring): one 32-bit word per (query row, 32-key tile).
+constexpr int kMaskWords = 20480;
+
+// Four mask bytes -> four keep bits (byte != 0), byte e in bit e.
+__device__ __forceinline__ uint32_t nonzero4(uint32_t x) {
+  const uint32_t y = (((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u) >> 7);
+  return (y | (y >> 7) | (y >> 14) | (y >> 21)) & 0xFu;
+}
+typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
+
 enum KernelMode : int { kModeAny = 0, kModeF32Paged = 1, kModeF32Dense = 2 };
 
 // A compile-time integer: the ring stage of an unrolled loop step, so that
@@ -180,7 +191,9 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   constexpr int PT_OFF = G::RING;
   constexpr int VIS_OFF = PT_OFF + kPageLds * 4;
   constexpr int VIS_W = BIG ? kTreeMaxW : kTreeNodeW;  // words per table entry
-  constexpr int LDS_BYTES = VIS_OFF + (BIG ? kTreeSlots : kTreeNodeM) * VIS_W * 8;
+  // The byte mask's keep bits take the place of the tree table (a byte-masked
+  // call has no tree split).
+  constexpr int LDS_BYTES = VIS_OFF + (DMASK ? kMaskWords * 4 : (BIG ? kTreeSlots : kTreeNodeM) * VIS_W * 8);
 
   // One LDS allocation so that the DMA ring sits at offset 0 (addresses < 64 KiB).
   __shared__ __attribute__((aligned(1024))) uint8_t smem[LDS_BYTES];
@@ -473,7 +486,7 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
 
   // Keep mask of the scores of tile t (tail keys, tree visibility, byte mask).
   // Bit v of a lane <-> key 4*lg + 8*(v/4) + v%4 of the tile.
-  auto mask_scores = [&](f32x16& s, int t) {
+  auto mask_scores = [&](f32x16& s, int t, uint32_t mword) {
     const int64_t kb = kstart + (int64_t)t * KT;
     const int64_t ke = causal ? min(kend, c0 + 1 + node_of) : kend;  // this row's key end
     const int lim = (int)max(min(ke - kb, (int64_t)KT), (int64_t)-KT) - 4 * lg;  // valid keys from 4*lg
@@ -491,18 +504,58 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
       keep &= (vb & 0xFu) | ((vb >> 4) & 0xF0u) | ((vb >> 8) & 0xF00u) | ((vb >> 12) & 0xF000u);
     }
     if constexpr (DMASK) {
-      const uint8_t* mrow = a.dmask + (int64_t)b * a.dm_sb + (int64_t)node_of * a.dm_sm;
-      const int64_t n0 = kb + 4 * lg;
-      uint32_t mb = 0;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t n = n0 + 8 * (v >> 2) + (v & 3);
-        mb |= (uint32_t)((n < a.dm_n) && (mrow[n * a.dm_sn] != 0)) << v;
-      }
-      keep &= rvalid ? mb : 0u;
+      const uint32_t vb = mword >> (4 * lg);
+      keep &= (vb & 0xFu) | ((vb >> 4) & 0xF0u) | ((vb >> 8) & 0xF00u) | ((vb >> 12) & 0xF000u);
     }
 #pragma unroll
     for (int v = 0; v < 16; ++v) s[v] = ((keep >> v) & 1u) ? s[v] : kNegInf;
+  };
+
+  // Byte mask: each wave turns its 32 rows' mask bytes into keep bits, one
+  // word per (row, tile), for a window of tiles that its share of the LDS
+  // holds (every tile of the split in most calls; refilled at a ring cycle
+  // otherwise).  The loop then reads one word per lane and tile, and a tile
+  // that every row of the wave keeps whole takes the unmasked path.  Loading
+  // the 16 bytes a lane needs inside the loop instead made every tile wait for
+  // all DMA in flight: 415 us a call against 139 us for 48 rows, 32 heads, 32000 keys
+  // (D = 128, f16).  The words of a row are an odd stride apart, so that 32
+  // rows read without bank conflicts.
+  int mw_stride = 1, mw_span = 4, mw_t0 = 0;
+  uint32_t* mw_lds = reinterpret_cast<uint32_t*>(smem + VIS_OFF);
+  auto fill_mask = [&](int t0) {
+    mw_t0 = t0;
+    const int nw = min(mw_span, ntiles - t0);  // words of this window per row
+    int lpr = 1;                               // lanes per row (a power of two)
+    while (lpr < 64 && lpr < nw) lpr <<= 1;
+    const int rpp = 64 / lpr, sub = lane & (lpr - 1);
+    const uint8_t* mb = a.dmask + (int64_t)b * a.dm_sb;
+    const bool unit = a.dm_sn == 1;
+    for (int r0 = 0; r0 < 32; r0 += rpp) {
+      const int r = r0 + lane / lpr;
+      const int node = __shfl(node_of, r & 31);
+      const uint8_t* mrow = mb + (int64_t)node * a.dm_sm;
+#pragma unroll 4
+      for (int w = sub; w < nw; w += lpr) {
+        const int64_t n0 = kstart + (int64_t)(t0 + w) * KT;
+        uint32_t bits = 0;
+        if (r < 32) {
+          if (unit && n0 + KT <= a.dm_n) {
+            const u32x4 x0 = *reinterpret_cast<const u32x4_a1*>(mrow + n0);
+            const u32x4 x1 = *reinterpret_cast<const u32x4_a1*>(mrow + n0 + 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bits |= (nonzero4(x0[e]) << (4 * e)) | (nonzero4(x1[e]) << (16 + 4 * e));
+          } else {
+            for (int e = 0; e < KT; ++e)
+              if (n0 + e < a.dm_n && mrow[(n0 + e) * a.dm_sn] != 0) bits |= 1u << e;
+          }
+          mw_lds[(wid * 32 + r) * mw_stride + w] = bits;
+        }
+      }
+    }
+    // Lanes read words that other lanes of this wave wrote.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
 
   // ---- ping-pong schedule ------------------------------------------------------
@@ -562,6 +615,8 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
     u32x4 kf[KS], vf[2][DT];
     u32x4 pk[2];
     if (wave_active) {
+      uint32_t mword = ~0u;  // this row's keep bits of tile k (byte mask)
+      if constexpr (DMASK) mword = mw_lds[(wid * 32 + lj) * mw_stride + (k - mw_t0)];
       // Operands of X_k, read now so that their latency hides behind Y_k
       // (past the last tile K(k+1) is a stale stage whose product is unused).
       // The V^T reads are spread over the two halves of the exponentials so
@@ -574,8 +629,8 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
       // masked; on other tiles a score above mx + kSumTau shows as a lane's
       // sum of this tile's probabilities above 2^kSumTau (inf included), and
       // only then is the tile redone against its maximum.
-      const bool masked = is_tree || DMASK || k >= nvis;
-      if (masked) mask_scores(s_cur, k);
+      const bool masked = is_tree || (DMASK && __ballot(mword != ~0u) != 0ull) || k >= nvis;
+      if (masked) mask_scores(s_cur, k, mword);
       auto rescale = [&]() {
         const float mt = xor32_max(max16(s_cur)) * scale_log2;
         if (__ballot(mt > mx + kRescaleTau) != 0ull) {
@@ -637,6 +692,12 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   if (ntiles > 0) issue_tile(IC<0>{}, 0);
   if (ntiles > 1) issue_tile(IC<1>{}, 1);
   if (ntiles > 2 && !v_wave) issue_tile(IC<2>{}, 2);
+  if constexpr (DMASK) {
+    const int nact = min(NW, (a.R - rb * (NW * 32) + 31) / 32);  // waves with rows
+    mw_stride = (kMaskWords / (32 * nact) - 1) | 1;
+    mw_span = mw_stride & ~3;
+    if (wave_active && ntiles > 0) fill_mask(0);
+  }
   // The Q fragments must be complete before the loop.  The compiler counts
   // only its own loads (the DMA is inline asm): left to itself it would place
   // the Q waits at their first use inside the loop, where each one waits for
@@ -671,6 +732,7 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
     }
   }
   for (int t0 = 0; t0 < ntiles; t0 += 4) {
+    if (DMASK && wave_active && t0 - mw_t0 >= mw_span) fill_mask(t0);
     step(IC<0>{}, t0);
     if (t0 + 1 < ntiles) step(IC<1>{}, t0 + 1);
     if (t0 + 2 < ntiles) step(IC<2>{}, t0 + 2);
@@ -750,11 +812,9 @@ hipError_t launch_t(const AttnArgs& a, hipStream_t s, hipEvent_t ev0, hipEvent_t
   const int mp = dma_mode<D>(a.pre), mt = a.has_tree ? dma_mode<D>(a.tree) : mp;
   const bool pp = a.pre.pt != nullptr, tp = a.has_tree ? a.tree.pt != nullptr : pp;
   const dim3 grid((unsigned)nblk), block(512);
-  if constexpr (!DMASK) {
-    if (mp == kFast32 && mt == kFast32 && pp == tp && !(a.has_tree && a.M > kTreeNodeM)) {
-      if (pp) return launch_k(attn_splitk_kernel<T, D, DMASK, kModeF32Paged>, grid, block, s, ev0, ev1, a);
-      return launch_k(attn_splitk_kernel<T, D, DMASK, kModeF32Dense>, grid, block, s, ev0, ev1, a);
-    }
+  if (mp == kFast32 && mt == kFast32 && pp == tp && !(a.has_tree && a.M > kTreeNodeM)) {
+    if (pp) return launch_k(attn_splitk_kernel<T, D, DMASK, kModeF32Paged>, grid, block, s, ev0, ev1, a);
+    return launch_k(attn_splitk_kernel<T, D, DMASK, kModeF32Dense>, grid, block, s, ev0, ev1, a);
   }
   if constexpr (!DMASK) {
     if (a.has_tree && a.M > kTreeNodeM)
