@@ -1414,6 +1414,7 @@ int dsv_lmhead_accept(int mode, const dsv_tensor* hidden, const dsv_tensor* weig
   lm.p_sm = a.p_sm;
   lm.inv_temp = a.inv_temp;
   lm.nblk = dsv::lmhead_blocks(V);
+  a.cus = device_cus();
   const size_t R = (size_t)T * M, parts = R * (size_t)lm.nblk;
   char* ws = static_cast<char*>(workspace);
   lm.rstat = reinterpret_cast<float4*>(ws);

@@ -195,11 +195,8 @@ struct BundleArgs {
 };
 
 // Arguments of the lm_head fused with the acceptance statistics.
-constexpr int kLmThreads = 256;            // 4 waves
-constexpr int kLmRB = 2;                   // 32-row vocabulary blocks per wave
 constexpr int kLmKS = 4;                   // 16-element MFMA sub-steps per step
-constexpr int kLmVocab = 128 * kLmRB;      // vocabulary rows per workgroup
-constexpr int kLmRows = 64;                // hidden rows per pass over W
+constexpr int kLmVocab = 256;              // vocabulary rows per workgroup
 constexpr int kLmK = 16 * kLmKS;           // reduction elements per step
 struct LmArgs {
   int mode;                                // 0 greedy, 1 typical

@@ -180,3 +180,22 @@ def test_typical_near_the_threshold_rechecked_from_the_written_logits(gpu, delta
         w_toks, w_ids, w_alen, w_next, w_id = oacc.typical_walk(lg[t], draft[t].numpy(), [-1], pos.numpy(), 8,
                                                                  temperature=temperature, eps=0.09, alpha=0.3)
         assert info[t].tolist() == [w_id, w_alen, w_next, len(w_ids)], f"tree {t}"
+
+
+# Rows at the edges of the 64-, 128-, 192- and 256-row passes, with a
+# vocabulary of more slices than half the CUs (fewer take smaller passes, as in
+# the tests above) and one that ends inside a slice; Dm of 1, 3 and 5 steps.
+@pytest.mark.parametrize("T,M,Dm", [(1, 65, 64), (2, 64, 192), (1, 129, 320), (3, 64, 64), (1, 193, 192), (2, 128, 64),
+                                    (1, 257, 192), (3, 100, 320)])
+@pytest.mark.parametrize("mode", ["greedy", "typical"])
+def test_rows_of_a_pass(gpu, T, M, Dm, mode):
+    V = 33001
+    print(f"[lmhead rows] T={T} M={M} Dm={Dm} V={V} {mode}", flush=True)
+    h, w, draft, pref, pos, md = _case(gpu, T, M, Dm, V, seed=M + Dm)
+    r = lmhead_tree_accept(h, w, draft, pref, pos, md + 2, mode=mode, return_next=True, return_logits=True)
+    torch.cuda.synchronize()
+    _check_logits(h.reshape(-1, Dm), w, r["logits"].reshape(-1, V))
+    want = tree_accept(r["logits"], draft, pref, pos, md + 2, mode=mode, return_next=True)
+    torch.cuda.synchronize()
+    for key in ("path", "tokens", "info", "next"):
+        assert torch.equal(r[key], want[key]), key
