@@ -35,12 +35,14 @@
 //       head entries is the row's result.  Other rows (flat rows, a large k,
 //       an undecided cut, NaN or +inf logits) are left to the radix kernel
 //       (status 2, with m).
-//   sample_radix_kernel   one workgroup per row left open: 8-bit radix
-//       selection over the order keys of y (count-weighted for top-k,
-//       mass-weighted for top-p); the kept set (keys at or above both bounds)
-//       is gathered into LDS, where the index bound in the cut's tie group and
-//       the draw are taken when it fits; otherwise the bound comes from index
-//       passes over the row and the sweep draws.
+//   sample_radix_kernel   one workgroup per row left open (16-bit logits: or
+//       per row): for 16-bit logits the counts of the row's bit patterns, with
+//       their exact masses; for f32 8-bit radix selection over the order keys
+//       of y (count-weighted for top-k, mass-weighted for top-p).  The kept set
+//       (keys at or above both bounds) is gathered into LDS, where the index
+//       bound in the cut's tie group and the draw are taken when it fits;
+//       otherwise the bound comes from index passes over the row and the sweep
+//       draws.
 //   sample_sweep_kernel   one workgroup per (row, vocabulary range) of the
 //       rows still open (f32 rows without top-p / top-k when rows are fewer
 //       than CUs):
@@ -168,11 +170,12 @@ __device__ __forceinline__ uint32_t draw_word(int64_t v, int i, int t, uint64_t 
 // G = -ln(-ln U), U = (w + 0.5) * 2^-32, in double (the definition).  Not
 // inlined: the filters leave it to few entries, and one copy keeps the
 // kernels small.
-__device__ __noinline__ double gumbel(uint32_t w) {
+__device__ __forceinline__ double gumbel_inline(uint32_t w) {
 #pragma clang fp contract(off)
   const double u = ((double)w + 0.5) * 0x1p-32;
   return -det_ln(-det_ln(u));
 }
+__device__ __noinline__ double gumbel(uint32_t w) { return gumbel_inline(w); }
 
 // fp32 estimate of gumbel(w).  -ln U from U for U < 1/2, else from
 // x = 1 - U = (~w + 0.5) 2^-32 (a series below 2^-7), so that -ln U keeps its
@@ -972,8 +975,14 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
     __syncthreads();
   };
 
-  // Attempt 0: the regions' head; attempts 1, 2: the histogram's heads.
-  for (int att = 0; att < 3; ++att) {
+  // Attempt 0: the regions' head; attempts 1, 2: the histogram's heads.  16-bit
+  // rows with top-p take attempt 0 only, and only heads of up to NT entries
+  // (sorted by rank): the radix kernel's count of their values decides the
+  // others sooner than a histogram, a gathered head and its bitonic sort (a
+  // call of 256 rows of 128256, a tenth of them open: 381 us with them, 150 us
+  // without).
+  const bool brief = sizeof(LT) == 2 && use_p;
+  for (int att = 0; att < (brief ? 1 : 3); ++att) {
     if (att == 1 && jsel[1] == -2) histogram_heads();
     const int js = jsel[att];
     if (js < 0) {
@@ -1035,6 +1044,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
       });
     }
     __syncthreads();
+    if (brief && ncand > (uint32_t)NT) break;  // uniform over the block
     const int n = min((int)ncand, kCap);
     // The counts chose the threshold; the gathered count decides whether the
     // head fits and holds k entries.
@@ -1181,34 +1191,93 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
   if (tid == 0) a.sel[row] = make_uint4(__float_as_uint(m), 0u, 0u, 2u);
 }
 
-// Radix selection for the rows the select kernel left open (status 2): the
-// top-k key, the top-p cut key and, in the cut's tie group, the index bound;
-// the kept set is then gathered and drawn here when it fits in LDS, else the
-// bounds go to the sweep kernel.
+// Counters of the 16-bit selection: one per bit pattern of the logits, 16 bits
+// each, two to an LDS word (128 KiB).
+constexpr int kVWords = 32768;
+constexpr int kVList = 16384;  // kept entries held in LDS
+
+// The logit of dtype LT whose order key (16 bits, ykey's order) is k, and the
+// order keys of both halves of a word.
 template <typename LT>
-__global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const AcceptArgs a) {
+__device__ __forceinline__ float key16_to_f(uint32_t k) {
+  return int_to_f<LT>((int)((k & 0x8000u) ? (k ^ 0x8000u) : (~k & 0xFFFFu)));
+}
+__device__ __forceinline__ uint32_t key16x2(uint32_t w) {
+  const s16x2 sgn = __builtin_bit_cast(s16x2, w) >> (short)15;  // 0xFFFF for negative halves
+  return w ^ (__builtin_bit_cast(uint32_t, sgn) | 0x80008000u);
+}
+
+// Exclusive prefix sum over the block's threads; total: the block's sum.
+template <typename T, int NT>
+__device__ __forceinline__ T block_excl(T v, T* scratch, T& total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  T incl = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const T x = __shfl_up(incl, o);
+    if (lane >= o) incl += x;
+  }
+  __syncthreads();
+  if (lane == 63) scratch[w] = incl;
+  __syncthreads();
+  T base = 0;
+  total = 0;
+  for (int k = 0; k < NT / 64; ++k) {
+    if (k < w) base += scratch[k];
+    total += scratch[k];
+  }
+  return base + incl - v;
+}
+
+// One workgroup per row, for the rows that the select kernel left open (status
+// 2) or for all (16-bit logits only): the top-k key, the top-p cut key and, in
+// the cut's tie group, the index bound; the kept set is then gathered and drawn
+// here when it fits in LDS, else the bounds go to the sweep kernel.
+// 16-bit logits: a row has few distinct bit patterns, so one pass counts them,
+// and the counts times the patterns' exact masses give the row maximum, L, the
+// cut and the k-th value: 55-65 us a row of 128256 whatever its shape (14 us of
+// it the counting pass, LDS atomics; the counters take 128 KiB, one row per CU).
+// The digit passes, which form the mass of every entry in double, took 206 us.
+// A counter that overflows shows as a total below V (each overflow loses 65535
+// or 65536); such rows take the digit passes below, as f32 rows do.
+template <typename LT>
+__global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const AcceptArgs a, int all) {
   const int64_t row = blockIdx.x;
-  const uint4 st = a.sel[row];
-  if (st.w != 2u) return;
+  constexpr bool k16 = sizeof(LT) == 2;
+  float m = 0.f;  // the row maximum of y (f32: from the select kernel)
+  if (!k16 || all == 0) {
+    const uint4 st = a.sel[row];
+    if (st.w != 2u) return;
+    m = __uint_as_float(st.x);
+  }
   const int t = (int)(row / a.M), i = (int)(row % a.M);
   const LT* x = reinterpret_cast<const LT*>(a.logits) + (int64_t)t * a.l_st + (int64_t)i * a.l_sm;
   const int V = (int)a.V;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int ND = key_digits<LT>();
   constexpr int NV = 16 / sizeof(LT);
   const Warp wp = make_warp(a.temperature);
-  const float m = __uint_as_float(st.x);  // the row maximum of y, from the select kernel
   int S = 63;
   for (int vv = V; vv > 0; vv >>= 1) --S;  // 63 - bitlen(V)
   const int64_t kk = (a.top_k > 0 && a.top_k < V) ? a.top_k : 0;
   const bool use_p = a.top_p_q != 0;
-  (void)kk;
+  constexpr int kList = k16 ? kVList : 2 * kCap;  // kept entries drawn here
 
   __shared__ uint64_t hist[256];
   __shared__ uint32_t res_u[4];
   __shared__ uint64_t res_q[4];
-  __shared__ uint64_t cand[kCap];
+  // 16-bit: the counters, then the distinct values; both: the kept indices and
+  // the estimates of their z.
+  __shared__ __align__(16) uint32_t raw[k16 ? kVWords : 2 * kList];
+  static_assert(2 * kList <= (k16 ? kVWords : 2 * kList), "indices and estimates fit");
+  uint32_t* const list = raw;
+  float* const zest = reinterpret_cast<float*>(raw + kList);
+  __shared__ uint32_t gtab[k16 ? kVWords / 64 : 1];  // 16-bit: distinct values before each group of 64 words
+  __shared__ uint64_t scan_q[kRadixThreads / 64];
+  __shared__ uint32_t scan_u[kRadixThreads / 64];
+  __shared__ float xthr_s;
   __shared__ uint32_t ncand, nk_lo;
   __shared__ double red_d[kRadixThreads / 64];
   __shared__ int red_i[kRadixThreads / 64];
@@ -1221,12 +1290,213 @@ __global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const Accep
     a.sel[row] = make_uint4(0u, 0u, 0u, 1u);
   };
 
+  uint32_t tk = 0, ystar = 0, istar = 0;
+  uint64_t above = 0, Tq = 0;
+  bool decided = false;
+  float xlow = 0.f;  // decided: the row's lowest logit with a kept y
+
+  // ---- 16-bit logits: counts of the row's bit patterns ---------------------------
+  if constexpr (k16) {
+    constexpr int kIt = kVWords / kRadixThreads;  // counter words per thread
+    constexpr uint32_t kInfKey = 0x8000u | (uint32_t)IntOrder<LT>::kInf;
+    constexpr uint32_t kNegInfKey = 0x7FFFu - (uint32_t)IntOrder<LT>::kInf;
+    for (int q = tid; q < kVWords / 4; q += kRadixThreads) reinterpret_cast<u32x4*>(raw)[q] = u32x4{0u, 0u, 0u, 0u};
+    if (tid == 0) res_u[0] = res_u[1] = 0xFFFFFFFFu;  // y keys of the cut and the k-th; [2], [3]: lowest logit keys
+    __syncthreads();
+    uint32_t pad = 0;  // entries past the row's end (counted as -inf)
+    row_sweep_words<LT, kRadixThreads>(x, 0, V, [&](int64_t v0, const u32x4& r) {
+      if (v0 + NV > V) pad += (uint32_t)min((int64_t)NV, v0 + NV - V);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const uint32_t k2 = key16x2(r[w]);
+        atomicAdd(&raw[(k2 & 0xFFFFu) >> 1], (k2 & 1u) ? 65536u : 1u);
+        atomicAdd(&raw[k2 >> 17], (k2 & 0x10000u) ? 65536u : 1u);
+      }
+    });
+    __syncthreads();
+    // Thread tid holds word wtop - 1024 it for it = 0 .. 31: with it, then the
+    // wave, then the lane, then a word's higher half first, the keys descend.
+    // A wave's word of one it is a group: 64 words, which most rows leave empty
+    // (a bf16 binade is one group), so that the loops below skip it.
+    uint32_t cw[kIt];
+    uint32_t nc = 0, kmax = 0;
+    const int wtop = kVWords - 1 - tid;
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+      cw[it] = raw[wtop - kRadixThreads * it];
+      nc += (cw[it] & 0xFFFFu) + (cw[it] >> 16);
+    }
+    // NaN and -inf do not count: their keys lie in the first and last words.
+    auto drop = [&](int it, uint32_t lo, uint32_t hi) {  // keys outside [lo, hi]
+      const uint32_t k = 2u * (uint32_t)(wtop - kRadixThreads * it);
+      if (k < lo || k > hi) cw[it] &= 0xFFFF0000u;
+      if (k + 1u < lo || k + 1u > hi) cw[it] &= 0xFFFFu;
+    };
+    static_assert(2 * (kVWords - kRadixThreads) <= (int)kInfKey && 2 * kRadixThreads > (int)kNegInfKey, "first and last words");
+    drop(0, 0u, kInfKey);
+    drop(kIt - 1, kNegInfKey + 1u, 0xFFFFu);
+#pragma unroll
+    for (int it = kIt - 1; it >= 0; --it)
+      if (cw[it] != 0u) kmax = 2u * (uint32_t)(wtop - kRadixThreads * it) + ((cw[it] >> 16) != 0u ? 1u : 0u);
+    uint32_t total = 0, npad = 0;
+    block_excl<uint32_t, kRadixThreads>(nc, scan_u, total);
+    block_excl<uint32_t, kRadixThreads>(pad, scan_u, npad);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o));
+    __syncthreads();
+    if (lane == 0) scan_u[tid >> 6] = kmax;
+    __syncthreads();
+    for (int w = 0; w < kRadixThreads / 64; ++w) kmax = max(kmax, scan_u[w]);
+    if (total != (uint32_t)V + npad) {
+      // A counter overflowed: the row maximum by a pass, then the digit passes.
+      m = thread_max<LT, kRadixThreads>(x, V);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+      __syncthreads();
+      if (lane == 0) scan_u[tid >> 6] = __float_as_uint(m);
+      __syncthreads();
+      for (int w = 0; w < kRadixThreads / 64; ++w) m = fmaxf(m, __uint_as_float(scan_u[w]));
+      if (m > kNegInfF) m = warp_y<LT>(f_to_raw<LT>(m), wp);
+    } else {
+      m = kmax > kNegInfKey ? warp_y<LT>(f_to_raw<LT>(key16_to_f<LT>(kmax)), wp) : kNegInfF;
+    }
+    if (!(m > kNegInfF)) {  // no finite logit: nothing is kept (token 0)
+      if (tid == 0) finish(0.0, -1);
+      return;
+    }
+    if (!use_p && kk == 0) {  // top-k of at least V: everything is kept
+      if (tid == 0) a.sel[row] = make_uint4(0u, 0u, 0u, 0u);
+      return;
+    }
+    // Values of the order from the maximum to the last that counts: -inf
+    // excluded, and with top-p the values whose mass surely rounds to 0.
+    const float yz = use_p ? m - (float)(S + 2) * 0x1.62e430p-1f : kNegInfF;
+    // A lower bound of their logits' keys: y = x / T rounded (2^-8) is at least
+    // yz only for x above xz.
+    uint32_t klow = kNegInfKey + 1u;
+    if (use_p && m < -kNegInfF) {
+      float xz = wp.T * yz;
+      xz -= fabsf(xz) * 0x1p-5f + (__is_same(LT, _Float16) ? 0x1p-13f : 0x1p-99f) * fmaxf(1.f, wp.T);
+      if (xz > kNegInfF)
+        klow = max(klow, __is_same(LT, _Float16)
+                             ? key16x2((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)xz)) & 0xFFFFu
+                             : key16x2(__float_as_uint(xz) >> 16) & 0xFFFFu);
+    }
+    // Distinct values of each group (group it of wave wv: number 16 it + wv).
+    constexpr int kWv = kRadixThreads / 64;
+    const int gtop = 2 * (kVWords - 1 - 64 * wv) + 1;  // the wave's first key at it = 0
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+      uint32_t n = 0;
+      if ((uint32_t)(gtop - 2 * kRadixThreads * it) >= klow) {  // uniform over the wave
+        drop(it, klow, 0xFFFFu);
+        n = (uint32_t)__popcll(__ballot((cw[it] >> 16) != 0u)) + (uint32_t)__popcll(__ballot((cw[it] & 0xFFFFu) != 0u));
+      } else {
+        cw[it] = 0u;
+      }
+      if (lane == 0) gtab[kWv * it + wv] = n;
+    }
+    __syncthreads();
+    uint32_t D = 0;
+    {
+      const uint32_t g = tid < kIt * kWv ? gtab[tid] : 0u;
+      const uint32_t ge = block_excl<uint32_t, kRadixThreads>(g, scan_u, D);
+      if (tid < kIt * kWv) gtab[tid] = ge;
+    }
+    __syncthreads();
+    if (total == (uint32_t)V + npad && D <= (uint32_t)kVWords) {  // uniform over the block
+      // The distinct values in descending order, (key << 16) | count, where
+      // the counters were (every thread holds its own in registers).
+      uint32_t* const vals = raw;
+#pragma unroll
+      for (int it = 0; it < kIt; ++it) {
+        const uint64_t bh = __ballot((cw[it] >> 16) != 0u), bl = __ballot((cw[it] & 0xFFFFu) != 0u);
+        if ((bh | bl) == 0ull) continue;
+        const uint64_t lt = (1ull << lane) - 1ull;
+        const uint32_t k = 2u * (uint32_t)(wtop - kRadixThreads * it);
+        uint32_t pos = gtab[kWv * it + wv] + (uint32_t)__popcll(bh & lt) + (uint32_t)__popcll(bl & lt);
+        if ((cw[it] >> 16) != 0u) vals[pos++] = ((k + 1u) << 16) | (cw[it] >> 16);
+        if ((cw[it] & 0xFFFFu) != 0u) vals[pos] = (k << 16) | (cw[it] & 0xFFFFu);
+      }
+      __syncthreads();
+      // Thread tid: values ept * tid .. + ept - 1, their masses and counts.
+      const int ept = ((int)D + kRadixThreads - 1) / kRadixThreads;
+      const int e0 = min(ept * tid, (int)D), e1 = min(e0 + ept, (int)D);
+      auto y_of = [&](uint32_t ve) { return warp_y<LT>(f_to_raw<LT>(key16_to_f<LT>(ve >> 16)), wp); };
+      uint64_t tq = 0;
+      uint32_t tc = 0;
+      for (int e = e0; e < e1; ++e) {
+        const uint32_t ve = vals[e];
+        if (use_p) tq += fixed_mass(y_of(ve), m, S) * (ve & 0xFFFFu);
+        tc += ve & 0xFFFFu;
+      }
+      uint64_t L = 0;
+      uint32_t call = 0;
+      uint64_t qa = block_excl<uint64_t, kRadixThreads>(tq, scan_q, L);
+      uint32_t ca = block_excl<uint32_t, kRadixThreads>(tc, scan_u, call);
+      const uint64_t target = use_p ? tq_of(a.top_p_q, L) : 0ull;
+      // The value the top-p mass is reached in (and the mass above every value
+      // of the same y: several logits can share one), and the k-th largest.
+      const bool has_p = use_p && qa < target && qa + tq >= target;
+      const bool has_k = kk > 0 && (uint64_t)ca < (uint64_t)kk && (uint64_t)ca + tc >= (uint64_t)kk;
+      if (has_p || has_k) {
+        bool need_p = has_p, need_k = has_k;
+        for (int e = e0; e < e1; ++e) {
+          const uint32_t ve = vals[e], cnt = ve & 0xFFFFu;
+          const float y = y_of(ve);
+          if (need_p) {
+            const uint64_t q1 = fixed_mass(y, m, S);
+            if (qa + q1 * cnt >= target) {
+              uint64_t ab = qa;
+              for (int f = e - 1; f >= 0 && y_of(vals[f]) == y; --f) ab -= q1 * (vals[f] & 0xFFFFu);
+              int g = e;
+              while (g + 1 < (int)D && y_of(vals[g + 1]) == y) ++g;
+              res_u[0] = ykey(y);
+              res_u[2] = vals[g] >> 16;
+              res_q[0] = ab;
+              need_p = false;
+            }
+            qa += q1 * cnt;
+          }
+          if (need_k && (uint64_t)ca + cnt >= (uint64_t)kk) {
+            int g = e;
+            while (g + 1 < (int)D && y_of(vals[g + 1]) == y) ++g;
+            res_u[1] = ykey(y);
+            res_u[3] = vals[g] >> 16;
+            need_k = false;
+          }
+          ca += cnt;
+        }
+      }
+      __syncthreads();
+      // A k beyond the counted entries passes every one of them (top-p: every
+      // entry that the cut keeps).
+      uint32_t kx = vals[D - 1] >> 16;  // key of the lowest logit that can be kept
+      if (use_p) kx = res_u[2];
+      if (res_u[1] != 0xFFFFFFFFu) {
+        tk = res_u[1];
+        kx = max(kx, res_u[3]);
+      } else if (!use_p) {
+        tk = ykey(y_of(vals[D - 1]));
+      }
+      xlow = key16_to_f<LT>(kx);
+      if (use_p) {
+        ystar = res_u[0];
+        above = res_q[0];
+        Tq = target;
+      }
+      decided = true;
+    }
+    __syncthreads();
+  }
+
   // ---- radix selection over the whole row -------------------------------------
 
   // One radix pass: histogram of digit `shift` over the elements whose key
   // matches `prefix` above that digit (and, for the tie pass, key == tie_key
   // with the index as the digit source), weighted by count or mass.
-  auto pass = [&](int shift, uint32_t prefix, bool mass, bool by_index, uint32_t tie_key) {
+  // (Inlined: a call would keep everything it captures in scratch memory.)
+  auto pass = [&](int shift, uint32_t prefix, bool mass, bool by_index, uint32_t tie_key) __attribute__((always_inline)) {
     if (tid < 256) hist[tid] = 0;
     __syncthreads();
     const uint32_t hi_mask = shift >= 24 ? 0u : ~((1u << (shift + 8)) - 1u);
@@ -1245,8 +1515,8 @@ __global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const Accep
   };
 
   // top-k: the k-th largest key (1-based rank, with multiplicity).
-  uint32_t tk = 0;
-  if (a.top_k > 0 && a.top_k < V) {
+  if (!decided && kk > 0) {
+    tk = 0;
     uint32_t prefix = 0;
     uint64_t rank = (uint64_t)a.top_k;
     for (int d = 0; d < ND; ++d) {
@@ -1270,9 +1540,8 @@ __global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const Accep
 
   // top-p: the key of the last kept element (ystar), then the index bound in
   // its tie group (istar).
-  uint32_t ystar = 0, istar = 0;
-  uint64_t above = 0, Tq = 0;
-  if (use_p) {
+  if (!decided && use_p) {
+    above = 0;
     uint32_t prefix = 0;
     for (int d = 0; d < ND; ++d) {
       const int shift = 24 - 8 * d;
@@ -1332,7 +1601,7 @@ __global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const Accep
   // The index bound among the tie members: the rank-th largest index, digit
   // by digit (8-bit digits over bitlen(V - 1) bits); count(shift, prefix)
   // fills hist with the digit counts of the members that match prefix above.
-  auto index_bound = [&](uint64_t rank, auto&& count) -> uint32_t {
+  auto index_bound = [&](uint64_t rank, auto&& count) __attribute__((always_inline)) -> uint32_t {
     int ib = 0;
     for (int vv = V - 1; vv > 0; vv >>= 1) ++ib;
     uint32_t ipre = 0;
@@ -1359,29 +1628,32 @@ __global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const Accep
   // When it fits, the tie bound and the draw are taken here; otherwise the
   // bounds go to the sweep kernel.
   {
+    // By the warper's monotony, key(y) >= lower is x >= x_thr on the logits.
     const uint32_t lower = max(tk, ystar);
-    uint32_t* list = reinterpret_cast<uint32_t*>(cand);  // kList indices
-    constexpr int kList = 2 * kCap;
+    if (tid < 64 && !decided) {
+      const float xt = x_threshold<LT>(key_to_y(lower), wp);
+      if (tid == 0) xthr_s = xt;
+    }
     if (tid == 0) ncand = 0;
     __syncthreads();
-    row_sweep<LT, kRadixThreads>(x, 0, V, wp, [&](int64_t v0, const float(&y)[NV]) {
-      bool any = false;
-#pragma unroll
-      for (int e = 0; e < NV; ++e) any |= v0 + e < V && ykey(y[e]) >= lower;
-      if (__ballot(any) == 0ull) return;
+    const float xthr = decided ? xlow : xthr_s;
+    row_sweep<LT, kRadixThreads, false, true>(x, 0, V, wp, [&](int64_t v0, const float(&xv)[NV]) {
+      uint64_t bal[NV];
+      uint32_t tot = 0;
 #pragma unroll
       for (int e = 0; e < NV; ++e) {
-        const bool c = v0 + e < V && ykey(y[e]) >= lower;
-        const uint64_t bal = __ballot(c);
-        if (bal != 0ull) {
-          uint32_t base = 0;
-          if (lane == 0) base = atomicAdd(&ncand, (uint32_t)__popcll(bal));
-          base = __shfl(base, 0);
-          if (c) {
-            const uint32_t slot = base + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-            if (slot < (uint32_t)kList) list[slot] = (uint32_t)(v0 + e);
-          }
-        }
+        bal[e] = __ballot(v0 + e < V && xv[e] >= xthr);
+        tot += (uint32_t)__popcll(bal[e]);
+      }
+      if (tot == 0u) return;
+      uint32_t slot = 0;
+      if (lane == 0) slot = atomicAdd(&ncand, tot);
+      slot = __shfl(slot, 0);
+#pragma unroll
+      for (int e = 0; e < NV; ++e) {
+        const uint32_t q = slot + (uint32_t)__popcll(bal[e] & ((1ull << lane) - 1ull));
+        if (((bal[e] >> lane) & 1ull) && q < (uint32_t)kList) list[q] = (uint32_t)(v0 + e);
+        slot += (uint32_t)__popcll(bal[e]);
       }
     });
     __syncthreads();
@@ -1412,18 +1684,37 @@ __global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const Accep
             __syncthreads();
           });
       }
-      double bz = -__builtin_huge_val();
-      int bi = -1;
+      // fp32 estimates of the kept entries' z, their best lower bound over the
+      // block, then the exact draw of the entries that can still reach it.
+      float lb = kNegInfF;
       for (int q = tid; q < nl; q += kRadixThreads) {
         const int v = (int)list[q];
         const float y = warp_y<LT>(x[v], wp);
         const uint32_t k = ykey(y);
+        float zf = kNegInfF;
         if (k >= tk && (k > ystar || (k == ystar && (uint32_t)v >= istar))) {
-          const double z = (double)y + gumbel(draw_word(v, i, t, a.seed));
-          if (bi < 0 || z > bz || (z == bz && v < bi)) {
-            bz = z;
-            bi = v;
-          }
+          zf = y + gumbel_est(draw_word(v, i, t, a.seed));
+          lb = fmaxf(lb, zf - (kZMargin + fabsf(zf) * kZMarginRel));
+        }
+        zest[q] = zf;
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) lb = fmaxf(lb, __shfl_xor(lb, o));
+      __syncthreads();
+      if (lane == 0) scan_u[tid >> 6] = __float_as_uint(lb);
+      __syncthreads();
+      for (int w = 0; w < kRadixThreads / 64; ++w) lb = fmaxf(lb, __uint_as_float(scan_u[w]));
+      double bz = -__builtin_huge_val();
+      int bi = -1;
+      for (int q = tid; q < nl; q += kRadixThreads) {
+        const float zf = zest[q];
+        // (an infinite estimate, from an infinite y, is always drawn exactly)
+        if (zf == kNegInfF || !(zf + (kZMargin + fabsf(zf) * kZMarginRel) >= lb || zf == __builtin_huge_valf())) continue;
+        const int v = (int)list[q];
+        const double z = (double)warp_y<LT>(x[v], wp) + gumbel_inline(draw_word(v, i, t, a.seed));
+        if (bi < 0 || z > bz || (z == bz && v < bi)) {
+          bz = z;
+          bi = v;
         }
       }
       block_argmax(bz, bi, red_d, red_i, kRadixThreads);
@@ -1917,7 +2208,21 @@ __global__ void __launch_bounds__(kTempThreads) __attribute__((amdgpu_waves_per_
 template <typename LT>
 hipError_t launch_sample_t(const AcceptArgs& a, hipStream_t s) {
   const unsigned rows = (unsigned)((int64_t)a.T * a.M);
-  if (a.sel != nullptr) {
+  // 16-bit rows go straight to the value counts (all) where that is the faster
+  // order.  Top-p: one round of rows (up to the CUs) of enough rows that some
+  // are open, the select kernel's time then adds to the open rows': 256 rows
+  // of 128256, a tenth open, 77 against 150 us (no row open: 52 against 36); more
+  // rows than CUs take a round each here: 512 rows, none open, 100 against 62 us.
+  // Top-k alone: long rows or one round (512 x 128256: 97 against 123 us; 64:
+  // 54 against 73; 512 x 32000: 66 against 53).
+  const int64_t ncu = a.cus > 0 ? a.cus : 256;
+  const bool all = sizeof(LT) == 2 && (a.top_p_q != 0 ? (int64_t)rows <= ncu && rows >= 32
+                                                      : a.V >= 65536 || (int64_t)rows <= ncu);
+  if (a.sel != nullptr && all) {
+    hipLaunchKernelGGL(sample_radix_kernel<LT>, dim3(rows), dim3(kRadixThreads), 0, s, a, 1);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  } else if (a.sel != nullptr) {
     // One workgroup per row: 1024 threads when the rows leave CUs idle, else
     // 512, so that each CU holds two rows and their serial phases overlap.
     if ((int64_t)rows >= 2 * (int64_t)(a.cus > 0 ? a.cus : 256))
@@ -1926,7 +2231,7 @@ hipError_t launch_sample_t(const AcceptArgs& a, hipStream_t s) {
       hipLaunchKernelGGL((sample_select_kernel<LT, 1024>), dim3(rows), dim3(1024), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(sample_radix_kernel<LT>, dim3(rows), dim3(kRadixThreads), 0, s, a);
+    hipLaunchKernelGGL(sample_radix_kernel<LT>, dim3(rows), dim3(kRadixThreads), 0, s, a, 0);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
