@@ -176,7 +176,10 @@ __device__ __forceinline__ float max16(const f32x16& s) {
 // run time).
 // BIG: trees of more than kTreeNodeM nodes (the tree split's visibility table
 // indexed by packed row instead of node).
-template <typename T, int D, bool DMASK, int MODE, bool BIG = false>
+// DIRECT: one dense prefix split (a.direct): the output is written here, and a
+// causal block reads only the keys that its rows see.  A variant of its own: the
+// tests for it in every call cost 0.7-1 us.
+template <typename T, int D, bool DMASK, int MODE, bool BIG = false, bool DIRECT = false>
 __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   using G = Geo<D>;
   constexpr int NW = 8;
@@ -210,8 +213,16 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   // so that neighbouring work items (row blocks of one split) share an XCD.
   const int nblk = gridDim.x;
   int w = ((nblk & 7) == 0) ? (blockIdx.x & 7) * (nblk >> 3) + (blockIdx.x >> 3) : blockIdx.x;
-  const int rb = w % a.n_rb;
+  int rb = w % a.n_rb;
   w /= a.n_rb;
+  if (DIRECT && a.causal != 0 && a.n_rb > a.G) {
+    // Row blocks with the most visible keys first: the blocks of a query head
+    // follow one another and their keys grow towards the head's end, so take
+    // the last block of every head, then the last but one, and so on.
+    const int base = a.n_rb / a.G, rem = a.n_rb % a.G;
+    const int g = rb < base * a.G ? rb % a.G : rb - base * a.G, j = rb < base * a.G ? rb / a.G : base;
+    rb = g * base + min(g, rem) + base + (g < rem ? 1 : 0) - 1 - j;
+  }
   const int split = w % a.s_total;
   w /= a.s_total;
   const int kvh = w % a.Hk;
@@ -233,13 +244,19 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
     kstart = (int64_t)split * a.kps;
     kend = min(kstart + a.kps, n_pre_b);
   }
+  const bool causal = a.causal != 0 && !is_tree;
+  const int64_t c0 = n_pre_b - a.M;
+  if (DIRECT && causal) {
+    // Keys past the last one that any row of the block sees are not read.
+    const int r0 = rb * (NW * 32), r1 = min(r0 + NW * 32, a.R) - 1;
+    const int mlast = r1 - r0 >= a.M || r1 % a.M < r0 % a.M ? a.M - 1 : r1 % a.M;
+    kend = min(kend, c0 + 1 + mlast);
+  }
   const int64_t nkeys = kend - kstart;
   const int ntiles = nkeys > 0 ? (int)((nkeys + KT - 1) / KT) : 0;
   const int nfull = nkeys > 0 ? (int)(nkeys / KT) : 0;  // tiles without tail keys
   // Causal prefix (bottom-right aligned): row m sees keys n <= c0 + m with
   // c0 = len - M.  Tiles below nvis are visible to every row.
-  const bool causal = a.causal != 0 && !is_tree;
-  const int64_t c0 = n_pre_b - a.M;
   int nvis = nfull;
   if (causal) {
     const int64_t v = c0 + 1 - kstart;
@@ -762,8 +779,10 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
       const f32x16 x = acc[dt];
-      const u32x2 val = {pack2<BF16>(x[4 * q4] * inv, x[4 * q4 + 1] * inv),
-                         pack2<BF16>(x[4 * q4 + 2] * inv, x[4 * q4 + 3] * inv)};
+      u32x2 val = {pack2<BF16>(x[4 * q4] * inv, x[4 * q4 + 1] * inv),
+                   pack2<BF16>(x[4 * q4 + 2] * inv, x[4 * q4 + 3] * inv)};
+      if (DIRECT && a.direct == 2)
+        val = u32x2{pack2<F16>(x[4 * q4] * inv, x[4 * q4 + 1] * inv), pack2<F16>(x[4 * q4 + 2] * inv, x[4 * q4 + 3] * inv)};
       const int c = 4 * dt + q4;
       *reinterpret_cast<u32x2*>(stage + lj * (2 * D) + ((c ^ (lj % CHR)) * 16) + 8 * lg) = val;
     }
@@ -782,6 +801,21 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   for (int k = 0; k < CHR / 2; ++k) {
     const int f = k * 64 + lane, r = f / CHR, i = f % CHR;
     chunk[k] = *reinterpret_cast<const u32x4*>(stage + r * (2 * D) + ((i ^ (r % CHR)) * 16));
+  }
+  if constexpr (DIRECT) {
+    // Lane r (and r + 32) knows row r's head and node.
+    const int h = kvh * a.G + (rvalid ? r_me / a.M : 0);
+    const int64_t off = b * a.o_sb + (int64_t)node_of * a.o_sm + h * a.o_sh;
+#pragma unroll
+    for (int k = 0; k < CHR / 2; ++k) {
+      const int f = k * 64 + lane, r = f / CHR, i = f % CHR;
+      const int64_t o = __shfl(off, r);
+      if (row0 + r < a.R) *reinterpret_cast<u32x4*>(a.out + o + i * 8) = chunk[k];
+    }
+    if (rvalid && lg == 0 && a.lse != nullptr)
+      a.lse[b * a.l_sb + (int64_t)node_of * a.l_sm + h * a.l_sh] =
+          ltot > 0.f ? (mx + __log2f(ltot)) * 0.69314718055994530942f : kNegInf;
+    return;
   }
 #pragma unroll
   for (int k = 0; k < CHR / 2; ++k) {
@@ -812,6 +846,12 @@ hipError_t launch_t(const AttnArgs& a, hipStream_t s, hipEvent_t ev0, hipEvent_t
   const int mp = dma_mode<D>(a.pre), mt = a.has_tree ? dma_mode<D>(a.tree) : mp;
   const bool pp = a.pre.pt != nullptr, tp = a.has_tree ? a.tree.pt != nullptr : pp;
   const dim3 grid((unsigned)nblk), block(512);
+  if constexpr (!DMASK) {
+    if (a.direct != 0) {
+      if (mp != kFast32 || pp || a.has_tree) return hipErrorInvalidValue;  // (the host's rule)
+      return launch_k(attn_splitk_kernel<T, D, DMASK, kModeF32Dense, false, true>, grid, block, s, ev0, ev1, a);
+    }
+  }
   if (mp == kFast32 && mt == kFast32 && pp == tp && !(a.has_tree && a.M > kTreeNodeM)) {
     if (pp) return launch_k(attn_splitk_kernel<T, D, DMASK, kModeF32Paged>, grid, block, s, ev0, ev1, a);
     return launch_k(attn_splitk_kernel<T, D, DMASK, kModeF32Dense>, grid, block, s, ev0, ev1, a);

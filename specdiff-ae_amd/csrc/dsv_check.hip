@@ -184,6 +184,15 @@ void check_kernel1(const AttnArgs& a, bool dmask, const AttnExtents& ex, Checker
             if (a.row_perm != nullptr) ck.range(ex.perm, elem_addr(a.row_perm, mi, 4), 4, "row_perm read");
             const int64_t prow = (((int64_t)split * a.B + b) * a.Hk + kvh) * a.R + r;
             ck.cond(prow < nrows_all, "partial row out of range");
+            if (a.direct != 0) {
+              const int h = kvh * a.G + g;
+              const uintptr_t o = elem_addr(a.out, b * a.o_sb + (int64_t)m * a.o_sm + (int64_t)h * a.o_sh, 2);
+              ck.cond((o & 15) == 0, "output row not 16-byte aligned");
+              ck.range(ex.out, o, 2 * D, "output write");
+              if (a.lse != nullptr)
+                ck.range(ex.lse, elem_addr(a.lse, b * a.l_sb + (int64_t)m * a.l_sm + (int64_t)h * a.l_sh, 4), 4, "lse write");
+              continue;
+            }
             ck.range(ex.ws, elem_addr(a.opart, prow * D, 2), 2 * D, "partial write");
             ck.range(ex.ws, (uintptr_t)(a.ml + prow), 8, "partial stats write");
           }
@@ -321,7 +330,7 @@ int emulate_attention(const AttnArgs& a, const MergeArgs& m, int D, bool dmask, 
     f32 ? check_kernel_f32<64>(a, dmask, ex, ck) : check_kernel1<64>(a, dmask, ex, ck);
   else
     ck.cond(false, "unsupported head_dim in emulation");
-  if (ck.ok) check_merge(m, ex, ck);
+  if (ck.ok && a.direct == 0) check_merge(m, ex, ck);
   if (n_checked) *n_checked = ck.n_checked;
   return ck.ok ? 0 : -1;
 }

@@ -89,6 +89,14 @@ struct AttnArgs {
   uint16_t* opart;         // [S, B, Hk, R, D] bf16 partial outputs, normalised per split
   float2* ml;              // [S, B, Hk, R] (running max in log2 units, sum)
   int s_total;             // n_splits + has_tree
+
+  // One split only (direct: 1 bf16, 2 f16 output; 0 otherwise): the kernel writes the output rows (16-bit,
+  // 16-byte aligned) and the LSE itself, and no merge follows.
+  int direct;
+  uint16_t* out;           // [B, M, H, D] via strides
+  int64_t o_sb, o_sm, o_sh;
+  float* lse;              // optional, natural-log LSE at (b, m, h)
+  int64_t l_sb, l_sm, l_sh;
 };
 
 // Arguments of the LSE merge kernel (kernel 3).
