@@ -474,7 +474,9 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   const float scale_log2 = a.scale_log2;
 
   f32x16 acc[DT];
-  float mx = kNegInf, lsum = 0.f;
+  // (Byte mask: rows past the end never ask for a rescale of the wave's rows;
+  // their scores are 0 or dropped.)
+  float mx = DMASK && !rvalid ? 0.f : kNegInf, lsum = 0.f;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
 
@@ -532,9 +534,9 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   // word per (row, tile), for a window of tiles that its share of the LDS
   // holds (every tile of the split in most calls; refilled at a ring cycle
   // otherwise).  The loop then reads one word per lane and tile, and a tile
-  // that every row of the wave keeps whole takes the unmasked path.  Loading
-  // the 16 bytes a lane needs inside the loop instead made every tile wait for
-  // all DMA in flight: 415 us a call against 139 us for 48 rows, 32 heads, 32000 keys
+  // that every row of the wave keeps whole is not masked.  Loading the 16 bytes
+  // a lane needs inside the loop instead made every tile wait for all DMA in
+  // flight: 416 us a call against 137 us for 48 rows, 32 heads, 32000 keys
   // (D = 128, f16).  The words of a row are an odd stride apart, so that 32
   // rows read without bank conflicts.
   int mw_stride = 1, mw_span = 4, mw_t0 = 0;
@@ -642,12 +644,14 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
 
       // ---- Y_k: online softmax of S(k) (log2 domain, lazy rescale) ----------
       // The exponentials run against the lagging row maximum mx.  The tile's
-      // own maximum is taken only where mx is not known yet or the tile is
-      // masked; on other tiles a score above mx + kSumTau shows as a lane's
-      // sum of this tile's probabilities above 2^kSumTau (inf included), and
-      // only then is the tile redone against its maximum.
-      const bool masked = is_tree || (DMASK && __ballot(mword != ~0u) != 0ull) || k >= nvis;
-      if (masked) mask_scores(s_cur, k, mword);
+      // own maximum is taken only where mx is not known yet, the tile is
+      // masked or the call is (a mask changes which keys a row keeps, not how
+      // its probabilities are scaled); on other tiles a score above mx + kSumTau
+      // shows as a lane's sum of this tile's probabilities above 2^kSumTau (inf
+      // included), and only then is the tile redone against its maximum.
+      const bool drops = is_tree || (DMASK && __ballot(mword != ~0u) != 0ull) || k >= nvis;
+      if (drops) mask_scores(s_cur, k, mword);
+      const bool masked = DMASK || drops;
       auto rescale = [&]() {
         const float mt = xor32_max(max16(s_cur)) * scale_log2;
         if (__ballot(mt > mx + kRescaleTau) != 0ull) {
