@@ -49,8 +49,15 @@ constexpr float kNegInf = -__builtin_huge_valf();
 // exponentials may lag the true max by up to this much (p <= 2^8).
 constexpr float kRescaleTau = 8.0f;
 // Tiles after the first skip their maximum unless a lane's probabilities sum
-// above 2^kSumTau: every probability then stays below 2^kSumTau.
-constexpr float kSumBound = 65536.0f;  // 2^kSumTau, kSumTau = 16
+// above 2^kSumTau: every probability then stays at or below 2^kSumTau, which
+// must not round to infinity in the probabilities' type (f16: 65520 does).
+// Above kRescaleTau, so that a tile over the bound is always rescaled.
+template <typename T>
+constexpr int kSumTau = 16;
+template <>
+constexpr int kSumTau<F16> = 15;
+template <typename T>
+constexpr float kSumBound = (float)(1 << kSumTau<T>);
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
@@ -689,7 +696,7 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
         return ts;
       };
       float ts = exps(true);
-      if (!masked && __ballot(!(ts <= kSumBound)) != 0ull) {
+      if (!masked && __ballot(!(ts <= kSumBound<T>)) != 0ull) {
         rescale();
         ts = exps(false);
       }

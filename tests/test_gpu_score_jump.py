@@ -14,7 +14,9 @@ import math
 import pytest
 import torch
 
+from diffspec_mi355x.runtime.attention_compat import flash_attn_with_kvcache
 from diffspec_mi355x.runtime.bundle_verifier import FusedBundleVerifier, PagedBundleVerifier
+from diffspec_mi355x.runtime.tree_attention import tree_verify
 
 pytestmark = pytest.mark.gpu
 
@@ -71,3 +73,23 @@ def test_byte_mask_jump(gpu, dtype, D, jump):
     _check(*FusedBundleVerifier(device="cuda").verify_bundle(q, k, v, [mask]), want, "dense")
     pool, pt = _paged(k, v)
     _check(*ver.verify_bundle_paged(q, pool, pt, [mask]), want, "paged")
+
+
+@pytest.mark.parametrize("jump", JUMPS)
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_unmasked_jump(gpu, dtype, D, jump):
+    print(f"[score jump] tree, flash {dtype} D={D} jump={jump}", flush=True)
+    q, k, v = _inputs(gpu, D, dtype, jump)
+    out, lse = flash_attn_with_kvcache(q, k, v, return_softmax_lse=True)
+    _check(out, lse.transpose(1, 2), _reference(q, k, v), "flash")
+    # The same prefix with a chain of M nodes after it, dense and paged; node 0
+    # sees the prefix and itself.
+    kt, vt = (torch.cat([x, x[:, :M]], dim=1) for x in (k, v))
+    parent = torch.arange(-1, M - 1, device=gpu)
+    want = [torch.cat(x, dim=1) for x in zip(*(_reference(q[:, m:m + 1], kt[:, :N + m + 1], vt[:, :N + m + 1])
+                                               for m in range(M)))]
+    _check(*tree_verify(q, kt, vt, N, parent.expand(B, M).contiguous()), want, "tree dense")
+    pad = (0, 0, 0, 0, 0, 16 - M)
+    pool, pt = _paged(*(torch.nn.functional.pad(x, pad) for x in (kt, vt)))
+    _check(*tree_verify(q, pool[0, 0], pool[0, 1], N, parent.expand(B, M).contiguous(), page_table=pt), want, "tree paged")
