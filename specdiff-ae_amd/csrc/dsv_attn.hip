@@ -781,6 +781,14 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   if (!wave_active) return;
   const float ltot = xor32_sum(lsum);
   const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
+  if constexpr (DIRECT) {
+    // A row without a visible key writes zeros, as the merge does for it: V
+    // rows that others see may be infinite or NaN, and 0 times those is NaN.
+    if (!(mx > kNegInf)) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
+    }
+  }
   constexpr int CHR = D / 8;  // 16-byte chunks per row
   static_assert(NW * 32 * D * 2 <= G::RING, "the partial rows of all waves fit the ring");
   uint8_t* stage = smem + wid * (32 * D * 2);
@@ -825,7 +833,7 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
     }
     if (rvalid && lg == 0 && a.lse != nullptr)
       a.lse[b * a.l_sb + (int64_t)node_of * a.l_sm + h * a.l_sh] =
-          ltot > 0.f ? (mx + __log2f(ltot)) * 0.69314718055994530942f : kNegInf;
+          mx > kNegInf && ltot > 0.f ? (mx + __log2f(ltot)) * 0.69314718055994530942f : kNegInf;
     return;
   }
 #pragma unroll

@@ -43,3 +43,24 @@ def test_one_split_output(gpu, dtype, M, N, D, causal):
                 rel = ((out[b, seen, h].double() - o[seen]).norm() / o[seen].norm()).item()
                 err = (lse[b, h, seen].double() - l[seen]).abs().max().item()
                 assert rel <= 1e-2 and err <= 2e-3, (b, h, rel, err)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("D", [64, 128])
+def test_rows_without_keys_beside_nonfinite_values(gpu, dtype, bad, D):
+    B, M, H, Hk, N = 16, 70, 32, 16, 96
+    print(f"[direct output] rows without keys {dtype} {bad} D={D}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(D)
+    q, k, v = (torch.randn(s, generator=g, device=gpu).to(dtype) for s in ((B, M, H, D), (B, N, Hk, D), (B, N, Hk, D)))
+    v[:, 3] = bad
+    lens = torch.arange(B, device=gpu) * 5 + 1  # up to 76: the first M - len rows see nothing
+    out, lse = flash_attn_with_kvcache(q, k, v, causal=True, cache_seqlens=lens, return_softmax_lse=True)
+    torch.cuda.synchronize()
+    for b in range(B):
+        n = int(lens[b])
+        first = max(0, M - n)  # row m sees keys up to n - M + m
+        assert (out[b, :first] == 0).all() and torch.isneginf(lse[b, :, :first]).all(), f"batch {b}"
+        assert torch.isfinite(lse[b, :, first:]).all(), f"batch {b}"
+        sees = n - M + torch.arange(M, device=gpu) >= 3
+        assert not torch.isfinite(out[b, sees]).any(), f"batch {b}"
