@@ -220,20 +220,22 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   // so that neighbouring work items (row blocks of one split) share an XCD.
   const int nblk = gridDim.x;
   int w = ((nblk & 7) == 0) ? (blockIdx.x & 7) * (nblk >> 3) + (blockIdx.x >> 3) : blockIdx.x;
-  int rb = w % a.n_rb;
-  w /= a.n_rb;
-  if (DIRECT && a.causal != 0 && a.n_rb > a.G) {
-    // Row blocks with the most visible keys first: the blocks of a query head
-    // follow one another and their keys grow towards the head's end, so take
-    // the last block of every head, then the last but one, and so on.
-    const int base = a.n_rb / a.G, rem = a.n_rb % a.G;
-    const int g = rb < base * a.G ? rb % a.G : rb - base * a.G, j = rb < base * a.G ? rb / a.G : base;
-    rb = g * base + min(g, rem) + base + (g < rem ? 1 : 0) - 1 - j;
+  int rb, split, kvh, b;
+  if (DIRECT && a.long_first == 2) {
+    int head;
+    deal_block(blockIdx.x, a.B * a.Hk, a.n_rb, head, rb);
+    split = 0;
+    kvh = head % a.Hk;
+    b = head / a.Hk;
+  } else {
+    rb = w % a.n_rb;
+    w /= a.n_rb;
+    split = w % a.s_total;
+    w /= a.s_total;
+    kvh = w % a.Hk;
+    b = w / a.Hk;
   }
-  const int split = w % a.s_total;
-  w /= a.s_total;
-  const int kvh = w % a.Hk;
-  const int b = w / a.Hk;
+  if (DIRECT && a.long_first != 0) rb = long_first_rb(rb, a.n_rb, a.G);
   const bool is_tree = a.has_tree && split == a.n_splits;
   const KvSrc src = is_tree ? a.tree : a.pre;
 

@@ -91,8 +91,11 @@ struct AttnArgs {
   int s_total;             // n_splits + has_tree
 
   // One split only (direct: 1 bf16, 2 f16 output; 0 otherwise): the kernel writes the output rows (16-bit,
-  // 16-byte aligned) and the LSE itself, and no merge follows.
+  // 16-byte aligned) and the LSE itself, and no merge follows.  long_first: row
+  // blocks of a causal call that see most keys first (long_first_rb), 1 in
+  // contiguous eighths, 2 dealt (deal_block).
   int direct;
+  int long_first;
   uint16_t* out;           // [B, M, H, D] via strides
   int64_t o_sb, o_sm, o_sh;
   float* lse;              // optional, natural-log LSE at (b, m, h)
