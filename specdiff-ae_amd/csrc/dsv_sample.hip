@@ -35,14 +35,16 @@
 //       head entries is the row's result.  Other rows (flat rows, a large k,
 //       an undecided cut, NaN or +inf logits) are left to the radix kernel
 //       (status 2, with m).
-//   sample_radix_kernel   one workgroup per row left open (16-bit logits: or
-//       per row): for 16-bit logits the counts of the row's bit patterns, with
-//       their exact masses; for f32 8-bit radix selection over the order keys
-//       of y (count-weighted for top-k, mass-weighted for top-p).  The kept set
-//       (keys at or above both bounds) is gathered into LDS, where the index
-//       bound in the cut's tie group and the draw are taken when it fits;
-//       otherwise the bound comes from index passes over the row and the sweep
-//       draws.
+//       16-bit rows take the regions' head only; where one round of the CUs holds
+//       the rows, the same kernel goes on with what it does not decide, and rows
+//       whose threads' maxima show that it will not are not tried.
+//   sample_radix_kernel   one workgroup per row left open (or per row): for
+//       16-bit logits the counts of the row's bit patterns, with their exact
+//       masses; for f32 8-bit radix selection over the order keys of y
+//       (count-weighted for top-k, mass-weighted for top-p).  The kept set (keys
+//       at or above both bounds) is gathered into LDS, where the index bound in
+//       the cut's tie group and the draw are taken when it fits; otherwise the
+//       bound comes from index passes over the row and the sweep draws.
 //   sample_sweep_kernel   one workgroup per (row, vocabulary range) of the
 //       rows still open (f32 rows without top-p / top-k when rows are fewer
 //       than CUs):
@@ -526,16 +528,28 @@ __device__ __forceinline__ float int_to_f(int b) {
     return raw_to_f<LT>(__builtin_bit_cast(LT, (uint16_t)b));
 }
 
+// Sixteen bytes at p (ANY: 2-byte aligned).
+template <bool ANY>
+__device__ __forceinline__ u32x4 load16(const void* p) {
+  typedef u32x4 any_t __attribute__((aligned(2)));
+  if constexpr (ANY)
+    return *reinterpret_cast<const any_t*>(p);
+  else
+    return *reinterpret_cast<const u32x4*>(p);
+}
+
 // This thread's maximum of the row's logits (NaN counts as -inf) over the
 // vectors row_sweep would hand it: two integer extremes per packed word, then
 // the float they stand for.  A thread that met a positive NaN (it would pass
-// for the maximum) redoes its vectors entry by entry.
-template <typename LT, int NT>
+// for the maximum) redoes its vectors entry by entry.  ANY: rows that are not
+// 16-byte aligned (an odd V) are loaded by vectors too (64 rows of 50257 entry
+// by entry: 8 us more).
+template <typename LT, int NT, bool ANY = false>
 __device__ __forceinline__ float thread_max(const LT* x, int64_t hi) {
   constexpr int N = 16 / sizeof(LT);
   constexpr int64_t kStep = (int64_t)NT * N;
   using IO = IntOrder<LT>;
-  const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  const bool aligned = ANY || (reinterpret_cast<uintptr_t>(x) & 15) == 0;
   const int64_t first = (int64_t)threadIdx.x * N;
   auto word = [&](int64_t v0, int w) -> uint32_t {  // entries past hi read as -inf
     if constexpr (sizeof(LT) == 4) {
@@ -558,14 +572,14 @@ __device__ __forceinline__ float thread_max(const LT* x, int64_t hi) {
     for (; aligned && v0 + 3 * kStep + N <= hi; v0 += 4 * kStep) {
       u32x4 r[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) r[u] = *reinterpret_cast<const u32x4*>(x + v0 + u * kStep);
+      for (int u = 0; u < 4; ++u) r[u] = load16<ANY>(x + v0 + u * kStep);
 #pragma unroll
       for (int u = 0; u < 4; ++u) take(r[u]);
     }
     for (; v0 < hi; v0 += kStep) {
       u32x4 r;
       if (aligned && v0 + N <= hi)
-        r = *reinterpret_cast<const u32x4*>(x + v0);
+        r = load16<ANY>(x + v0);
       else
         r = u32x4{word(v0, 0), word(v0, 1), word(v0, 2), word(v0, 3)};
       take(r);
@@ -587,14 +601,14 @@ __device__ __forceinline__ float thread_max(const LT* x, int64_t hi) {
     for (; aligned && v0 + 3 * kStep + N <= hi; v0 += 4 * kStep) {
       u32x4 r[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) r[u] = *reinterpret_cast<const u32x4*>(x + v0 + u * kStep);
+      for (int u = 0; u < 4; ++u) r[u] = load16<ANY>(x + v0 + u * kStep);
 #pragma unroll
       for (int u = 0; u < 4; ++u) take(r[u]);
     }
     for (; v0 < hi; v0 += kStep) {
       u32x4 r;
       if (aligned && v0 + N <= hi)
-        r = *reinterpret_cast<const u32x4*>(x + v0);
+        r = load16<ANY>(x + v0);
       else
         r = u32x4{word(v0, 0), word(v0, 1), word(v0, 2), word(v0, 3)};
       take(r);
@@ -698,16 +712,36 @@ constexpr int kBins = kNTheta + 1;
 // so {a >= -theta} is a head of the order, held by the regions when theta <=
 // the smallest g of the waves.
 constexpr float kPreG0 = 16.f, kPreGMin = 2.f;
+// What a row's maxima must show for its regions' head to be tried (COUNT below):
+// heads of up to kTryHead entries (a larger one leaves entries so light at the
+// cut that the bounds of L rarely decide it; rows below kTryShort entries, whose
+// passes take little, try 1024), below which the order holds kTailMass times
+// as many entries of the last one's mass.  Simulated rows (N(0, 2.5-3.5) logits,
+// T 0.7-1, top-p 0.9-0.95, 32000 to 128256 entries): of 720 without a planted token
+// 1 is tried in vain, of 300 with 40 likely tokens 3, and 9 of those are not
+// tried; 1024 entries and 3 times instead try 18 of the 720 in vain.
+constexpr float kTryHead = 256.f, kTailMass = 4.f;
+constexpr int kTryShort = 16384;
 constexpr int kPre = 2048;  // entries of the regions of a block
 
+template <typename LT, int NT, typename F>
+__device__ __forceinline__ void row_sweep_words(const LT* x, int64_t lo, int64_t hi, F&& f);
+template <typename LT>
+constexpr int kRadixWords = sizeof(LT) == 2 ? 32768 : 4 * kCap;  // LDS words of radix_row
+template <typename LT>
+__device__ __forceinline__ void radix_row(const AcceptArgs& a, int64_t row, float m, uint32_t* raw);
+
 // Four waves per SIMD (at most 128 VGPRs): two 512-thread rows share a CU.
-template <typename LT, int NT>
+// COUNT (16-bit logits): the regions' head only, if it has up to NT entries; the
+// rows that it does not decide, or that show beforehand that it will not, take
+// the radix kernel's way here (in its LDS: these rows are done with theirs).
+template <typename LT, int NT, bool COUNT = false>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sample_select_kernel(const AcceptArgs a) {
   static_assert(kCap % NT == 0, "candidates split evenly over the threads");
   constexpr int kWaves = NT / 64;
-  constexpr int kHistWords = kWaves * kBins * 64;
+  constexpr int kHistWords = COUNT ? 2 * kPre : kWaves * kBins * 64;
   constexpr int kPreCap = kPre / kWaves;  // entries of a wave's region of pre
-  static_assert(kHistWords >= 2 * kCap && kCap >= 2 * NT, "the candidates (and a sorted copy of up to NT) fit where the histograms were");
+  static_assert(kHistWords >= (COUNT ? 2 * kPre : 2 * kCap) && kHistWords >= 4 * NT && kCap >= 2 * NT, "the candidates (and a sorted copy of up to NT) fit where the histograms were");
   const int64_t row = blockIdx.x;
   const int t = (int)(row / a.M), i = (int)(row % a.M);
   const LT* x = reinterpret_cast<const LT*>(a.logits) + (int64_t)t * a.l_st + (int64_t)i * a.l_sm;
@@ -721,8 +755,12 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
   // do not hold the cut), and the head's candidates ((key << 32) | index).
   // pre: the waves' regions of entries near the maximum, (index << 32) | bits
   // of y.
-  __shared__ __align__(16) uint32_t hist[kHistWords];
-  __shared__ __align__(16) uint64_t pre[kPre];
+  __shared__ __align__(16) uint32_t raw[COUNT ? kRadixWords<LT> : 1];
+  __shared__ __align__(16) uint32_t own_hist[COUNT ? 1 : kHistWords];
+  __shared__ __align__(16) uint64_t own_pre[COUNT ? 1 : kPre];
+  static_assert(!COUNT || kHistWords + 2 * kPre <= kRadixWords<LT>, "hist and pre lie in the radix kernel's LDS");
+  uint32_t* const hist = COUNT ? raw : own_hist;
+  uint64_t* const pre = COUNT ? reinterpret_cast<uint64_t*>(raw + kHistWords) : own_pre;
   uint64_t* cand = reinterpret_cast<uint64_t*>(hist);
   __shared__ float red_f[kWaves];
   __shared__ uint32_t pre_n[kWaves];
@@ -739,7 +777,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
 
   // Row maximum of y: the warper is monotone, so it is the warped maximum
   // logit (xm).
-  float m = thread_max<LT, NT>(x, V);
+  const float mine_x = thread_max<LT, NT, COUNT>(x, V);
+  float m = mine_x;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
   if (lane == 0) red_f[wv] = m;
@@ -771,7 +810,9 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
     if (tid == 0) a.sel[row] = make_uint4(0u, 0u, 0u, 0u);
     return;
   }
+  do {  // (left by break: COUNT, the row goes to radix_row below)
   if (!(m < -kNegInfF)) {  // +inf maximum: the radix kernel's exact masses
+    if constexpr (COUNT) break;
     if (tid == 0) a.sel[row] = make_uint4(__float_as_uint(m), 0u, 0u, 2u);
     return;
   }
@@ -786,10 +827,37 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
     nk_lo = 0;
     nk_hi = 0;
   }
-  __syncthreads();
   const float mc = m * 0x1.715476p+0f;
   // a of a logit's warped value: the one fp32 expression used for every decision on a.
   auto a_of = [&](float y) { return fmaf(y, 0x1.715476p+0f, -mc); };
+  if constexpr (COUNT) {
+    // The threads' maxima are a sample of the row: if N entries lie within some
+    // a, 1 - e^(-N / threads) of the threads have one there.  Top-k alone: the
+    // regions surely hold k entries if k maxima lie within their bound.  Top-p:
+    // a head of that many entries carries the mass if what lies below it is at
+    // most 1 - top_p of the maxima's mass; the a at which that holds must be
+    // reached by no more threads than that many entries reach.
+    const float am = a_of(warp_y<LT>(f_to_raw<LT>(mine_x), wp));  // -inf: no entry
+    float ms = am >= -kPreG0 ? __builtin_amdgcn_exp2f(am) : 0.f;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) ms += __shfl_xor(ms, o);
+    if (lane == 0) pre_g[wv] = ms;
+    __syncthreads();
+    ms = 0.f;
+    for (int w = 0; w < kWaves; ++w) ms += pre_g[w];
+    const float head = V < kTryShort ? 1024.f : kTryHead;
+    float alim = kPreG0;
+    if (use_p) alim = fminf(alim, __log2f(kTailMass * head / ((1.f - (float)a.top_p_q * 0x1p-32f) * ms)));
+    const uint32_t mcnt = (uint32_t)__popcll(__ballot(am >= -alim));
+    if (lane == 0) pre_n[wv] = mcnt;
+    __syncthreads();
+    uint32_t reach = 0;
+    for (int w = 0; w < kWaves; ++w) reach += pre_n[w];
+    const float active = (float)min((V + NV - 1) / NV, NT);  // threads with entries
+    if (use_p ? (float)reach > active * (1.f - __builtin_amdgcn_exp2f(-1.442695f * head / active)) : reach < (uint64_t)kk)
+      break;
+  }
+  __syncthreads();
   uint64_t* pw = pre + wv * kPreCap;
   // Per-wave bins of the appended entries (count of bin b at wbin_c[wv][b],
   // fp32 mass at wbin_q[wv][b]); bins past the final bound also count entries
@@ -872,6 +940,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
     gcov = fminf(gcov, pre_g[w]);
   }
   if (use_p && !(L == L)) {  // NaN logits (NaN counts as -inf): the radix kernel
+    if constexpr (COUNT) break;
     if (tid == 0) a.sel[row] = make_uint4(__float_as_uint(m), 0u, 0u, 2u);
     return;
   }
@@ -976,14 +1045,15 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
   };
 
   // Attempt 0: the regions' head; attempts 1, 2: the histogram's heads.  16-bit
-  // rows with top-p take attempt 0 only, and only heads of up to NT entries
-  // (sorted by rank): the radix kernel's count of their values decides the
-  // others sooner than a histogram, a gathered head and its bitonic sort (a
-  // call of 256 rows of 128256, a tenth of them open: 381 us with them, 150 us
-  // without).
-  const bool brief = sizeof(LT) == 2 && use_p;
+  // rows with top-p (COUNT: all) take attempt 0 only, and only heads of up to NT
+  // entries (sorted by rank): the count of their values decides the others
+  // sooner than a histogram, a gathered head and its bitonic sort (512 rows of
+  // 128256, a tenth of them open: 451 us a call with them, 170 us without).
+  const bool brief = COUNT || (sizeof(LT) == 2 && use_p);
   for (int att = 0; att < (brief ? 1 : 3); ++att) {
-    if (att == 1 && jsel[1] == -2) histogram_heads();
+    if constexpr (!COUNT) {
+      if (att == 1 && jsel[1] == -2) histogram_heads();
+    }
     const int js = jsel[att];
     if (js < 0) {
       if (att == 0) continue;
@@ -995,7 +1065,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
       nk_hi = 0;
     }
     if (att == 2) __syncthreads();
-    if (js >= kNTheta) {
+    if (COUNT || js >= kNTheta) {
       // From the waves' regions: the head {a > -kTheta[j]} (bins 0..j).
       const float ath = -kTheta[js - kNTheta];
       for (int q0 = 0; q0 < kPre; q0 += NT) {
@@ -1044,7 +1114,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
       });
     }
     __syncthreads();
-    if (brief && ncand > (uint32_t)NT) break;  // uniform over the block
+    if (brief && ncand > (uint32_t)NT) break;  // uniform over the block (at most kPre entries gathered)
     const int n = min((int)ncand, kCap);
     // The counts chose the threshold; the gathered count decides whether the
     // head fits and holds k entries.
@@ -1053,7 +1123,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
     // carry the index) into cand[NT, 2 NT); more by a bitonic sort in place,
     // padded with zero keys to a power of two.
     const uint64_t* keys = cand;
-    if (n <= NT) {
+    if (COUNT || n <= NT) {
       uint64_t* out = cand + NT;  // above the n <= NT candidates
       if (tid < n) {
         const uint64_t mine = cand[tid];
@@ -1186,9 +1256,15 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
     }
     __syncthreads();
   }
+  } while (false);
 
-  // ---- not decided here: the radix kernel takes the row (status 2, with m) --
-  if (tid == 0) a.sel[row] = make_uint4(__float_as_uint(m), 0u, 0u, 2u);
+  // ---- not decided here ---------------------------------------------------------
+  if constexpr (COUNT) {
+    __syncthreads();  // the row's LDS above is read no more
+    radix_row<LT>(a, row, m, raw);
+  } else {  // the radix kernel takes the row (status 2, with m)
+    if (tid == 0) a.sel[row] = make_uint4(__float_as_uint(m), 0u, 0u, 2u);
+  }
 }
 
 // Counters of the 16-bit selection: one per bit pattern of the logits, 16 bits
@@ -1240,16 +1316,12 @@ __device__ __forceinline__ T block_excl(T v, T* scratch, T& total) {
 // The digit passes, which form the mass of every entry in double, took 206 us.
 // A counter that overflows shows as a total below V (each overflow loses 65535
 // or 65536); such rows take the digit passes below, as f32 rows do.
+// (m: the row maximum of y; 16-bit logits: not read.  raw: kRadixWords<LT> LDS words.)
 template <typename LT>
-__global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const AcceptArgs a, int all) {
-  const int64_t row = blockIdx.x;
+constexpr int kRadixList = sizeof(LT) == 2 ? kVList : 2 * kCap;  // kept entries drawn here
+template <typename LT>
+__device__ __forceinline__ void radix_row(const AcceptArgs& a, int64_t row, float m, uint32_t* raw) {
   constexpr bool k16 = sizeof(LT) == 2;
-  float m = 0.f;  // the row maximum of y (f32: from the select kernel)
-  if (!k16 || all == 0) {
-    const uint4 st = a.sel[row];
-    if (st.w != 2u) return;
-    m = __uint_as_float(st.x);
-  }
   const int t = (int)(row / a.M), i = (int)(row % a.M);
   const LT* x = reinterpret_cast<const LT*>(a.logits) + (int64_t)t * a.l_st + (int64_t)i * a.l_sm;
   const int V = (int)a.V;
@@ -1263,15 +1335,14 @@ __global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const Accep
   for (int vv = V; vv > 0; vv >>= 1) --S;  // 63 - bitlen(V)
   const int64_t kk = (a.top_k > 0 && a.top_k < V) ? a.top_k : 0;
   const bool use_p = a.top_p_q != 0;
-  constexpr int kList = k16 ? kVList : 2 * kCap;  // kept entries drawn here
+  constexpr int kList = kRadixList<LT>;
 
   __shared__ uint64_t hist[256];
   __shared__ uint32_t res_u[4];
   __shared__ uint64_t res_q[4];
-  // 16-bit: the counters, then the distinct values; both: the kept indices and
-  // the estimates of their z.
-  __shared__ __align__(16) uint32_t raw[k16 ? kVWords : 2 * kList];
-  static_assert(2 * kList <= (k16 ? kVWords : 2 * kList), "indices and estimates fit");
+  // raw: for 16-bit logits the counters, then the distinct values; for both the
+  // kept indices and the estimates of their z.
+  static_assert(2 * kList <= kRadixWords<LT>, "indices and estimates fit");
   uint32_t* const list = raw;
   float* const zest = reinterpret_cast<float*>(raw + kList);
   __shared__ uint32_t gtab[k16 ? kVWords / 64 : 1];  // 16-bit: distinct values before each group of 64 words
@@ -1744,6 +1815,19 @@ __global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const Accep
   if (tid == 0) a.sel[row] = make_uint4(tk, ystar, istar, 0u);
 }
 
+template <typename LT>
+__global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const AcceptArgs a, int all) {
+  __shared__ __align__(16) uint32_t raw[kRadixWords<LT>];
+  const int64_t row = blockIdx.x;
+  float m = 0.f;
+  if (sizeof(LT) != 2 || all == 0) {
+    const uint4 st = a.sel[row];
+    if (st.w != 2u) return;
+    m = __uint_as_float(st.x);
+  }
+  radix_row<LT>(a, row, m, raw);
+}
+
 // Gumbel-max draw over one vocabulary range of one row.
 template <typename LT>
 __global__ void __launch_bounds__(kSweepThreads) sample_sweep_kernel(const AcceptArgs a) {
@@ -2208,17 +2292,26 @@ __global__ void __launch_bounds__(kTempThreads) __attribute__((amdgpu_waves_per_
 template <typename LT>
 hipError_t launch_sample_t(const AcceptArgs& a, hipStream_t s) {
   const unsigned rows = (unsigned)((int64_t)a.T * a.M);
-  // 16-bit rows go straight to the value counts (all) where that is the faster
-  // order.  Top-p: one round of rows (up to the CUs) of enough rows that some
-  // are open, the select kernel's time then adds to the open rows': 256 rows
-  // of 128256, a tenth open, 77 against 150 us (no row open: 52 against 36); more
-  // rows than CUs take a round each here: 512 rows, none open, 100 against 62 us.
-  // Top-k alone: long rows or one round (512 x 128256: 97 against 123 us; 64:
-  // 54 against 73; 512 x 32000: 66 against 53).
+  // 16-bit rows of one round of the CUs: the regions' head, else the value counts,
+  // in one kernel.  (Microseconds of a call on rows that are all sure of their
+  // token / of which a tenth share the mass between thousands; 64 rows, top-p 0.9.
+  // 128256 entries: 46 / 76, counts alone 52 / 72, heads and histograms first 49 /
+  // 360; 32000: 27 / 46, 38 / 43, 31 / 162.)
+  // Straight to the counts (all) where the row maximum that comes before a head
+  // costs more than a head saves: top-k alone from 65536 entries (64 rows: 53 on
+  // sure rows, 58 with heads tried first, 128 with heads and histograms; 512 rows
+  // 98 and 218), and bf16 rows of that length that fill three quarters of the CUs,
+  // whose passes are bound by memory (256 rows: 55 / 74, 52 / 82, 56 / 376; f16 rows
+  // count slower: 65 / 86, 57 / 94, 61 / 486).  More rows than CUs would take a round
+  // each in the counts: 512 rows, none open, 100 against 83.
   const int64_t ncu = a.cus > 0 ? a.cus : 256;
-  const bool all = sizeof(LT) == 2 && (a.top_p_q != 0 ? (int64_t)rows <= ncu && rows >= 32
-                                                      : a.V >= 65536 || (int64_t)rows <= ncu);
-  if (a.sel != nullptr && all) {
+  const bool k16 = sizeof(LT) == 2, fits = (int64_t)rows <= ncu, full = 4 * (int64_t)rows >= 3 * ncu;
+  const bool all = k16 && a.V >= 65536 && (a.top_p_q == 0 || (__is_same(LT, uint16_t) && fits && full));
+  if (a.sel != nullptr && k16 && fits && !all) {
+    if constexpr (sizeof(LT) == 2) hipLaunchKernelGGL((sample_select_kernel<LT, kRadixThreads, true>), dim3(rows), dim3(kRadixThreads), 0, s, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  } else if (a.sel != nullptr && all) {
     hipLaunchKernelGGL(sample_radix_kernel<LT>, dim3(rows), dim3(kRadixThreads), 0, s, a, 1);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
