@@ -141,10 +141,6 @@ __device__ __forceinline__ bool tmask_keep(const AttnArgs& a, int b, int i, int 
   }
 }
 
-// LDS words of the byte-mask variant's keep-bit window (80 KiB beside the
-// ring): one 32-bit word per (query row, 32-key tile).
-constexpr int kMaskWords = 20480;
-
 // Four mask bytes -> four keep bits (byte != 0), byte e in bit e.
 __device__ __forceinline__ uint32_t nonzero4(uint32_t x) {
   const uint32_t y = (((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u) >> 7);
@@ -256,10 +252,7 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   const bool causal = a.causal != 0 && !is_tree;
   const int64_t c0 = n_pre_b - a.M;
   if (DIRECT && causal) {
-    // Keys past the last one that any row of the block sees are not read.
-    const int r0 = rb * (NW * 32), r1 = min(r0 + NW * 32, a.R) - 1;
-    const int mlast = r1 - r0 >= a.M || r1 % a.M < r0 % a.M ? a.M - 1 : r1 % a.M;
-    kend = min(kend, c0 + 1 + mlast);
+    kend = causal_kend(rb, NW * 32, a.M, a.R, c0, kend);
   }
   const int64_t nkeys = kend - kstart;
   const int ntiles = nkeys > 0 ? (int)((nkeys + KT - 1) / KT) : 0;
@@ -723,9 +716,8 @@ __global__ void __launch_bounds__(512, 2) attn_splitk_kernel(const AttnArgs a) {
   if (ntiles > 1) issue_tile(IC<1>{}, 1);
   if (ntiles > 2 && !v_wave) issue_tile(IC<2>{}, 2);
   if constexpr (DMASK) {
-    const int nact = min(NW, (a.R - rb * (NW * 32) + 31) / 32);  // waves with rows
-    mw_stride = (kMaskWords / (32 * nact) - 1) | 1;
-    mw_span = mw_stride & ~3;
+    mw_stride = mask_stride(mask_waves(rb, NW, a.R));
+    mw_span = mask_span(mw_stride);
     if (wave_active && ntiles > 0) fill_mask(0);
   }
   // The Q fragments must be complete before the loop.  The compiler counts

@@ -157,6 +157,27 @@ DSV_HD void deal_block(int p, int heads, int n_rb, int& head, int& i) {
   }
 }
 
+// Key end of row block rb of a causal one-split call: keys past the last one
+// that any of its rows (r = head * M + node) sees are not read.
+DSV_HD int64_t causal_kend(int rb, int rows_per_block, int M, int R, int64_t c0, int64_t kend) {
+  const int r0 = rb * rows_per_block, r1 = (r0 + rows_per_block < R ? r0 + rows_per_block : R) - 1;
+  const int mlast = r1 - r0 >= M || r1 % M < r0 % M ? M - 1 : r1 % M;
+  const int64_t e = c0 + 1 + mlast;
+  return e < kend ? e : kend;
+}
+
+// The byte-mask variant's keep-bit window: LDS words (80 KiB beside the ring),
+// one 32-bit word per (query row, 32-key tile); the words of a row are an odd
+// stride apart, for the waves of row block rb that have rows, and a window spans
+// whole ring cycles of four tiles.
+constexpr int kMaskWords = 20480;
+DSV_HD int mask_waves(int rb, int waves, int R) {
+  const int n = (R - rb * (waves * 32) + 31) / 32;
+  return n < waves ? n : waves;
+}
+DSV_HD int mask_stride(int active_waves) { return (kMaskWords / (32 * active_waves) - 1) | 1; }
+DSV_HD int mask_span(int stride) { return stride & ~3; }
+
 DSV_HD int64_t clamp_page(int64_t pg, int64_t n_phys) { return pg < 0 ? 0 : (pg >= n_phys ? n_phys - 1 : pg); }
 
 }  // namespace dsv

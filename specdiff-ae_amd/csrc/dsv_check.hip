@@ -11,6 +11,7 @@
 
 #include <cstdio>
 #include <string>
+#include <vector>
 
 #include "dsv_attn_f32_geo.h"
 #include "dsv_attn_geo.h"
@@ -57,6 +58,19 @@ void check_kernel1(const AttnArgs& a, bool dmask, const AttnExtents& ex, Checker
   using G = Geo<D>;
   const int RING = G::RING;
   ck.cond(RING <= 65536, "LDS-DMA ring above 64 KiB");
+  if (a.long_first != 0) {
+    // The sorted order meets every (head, row block) once.
+    ck.cond(a.direct != 0 && a.s_total == 1 && a.n_rb > 0, "sorted row blocks outside a one-split call");
+    const int heads = a.B * a.Hk;
+    std::vector<char> seen((size_t)heads * a.n_rb, 0);
+    for (int p = 0; p < heads * a.n_rb && ck.ok; ++p) {
+      int head = p / a.n_rb, i = p % a.n_rb;
+      if (a.long_first == 2) deal_block(p, heads, a.n_rb, head, i);
+      const int rb = long_first_rb(i, a.n_rb, a.G);
+      if (ck.cond(head >= 0 && head < heads && rb >= 0 && rb < a.n_rb, "row block out of range"))
+        ck.cond(seen[(size_t)head * a.n_rb + rb]++ == 0, "row block met twice");
+    }
+  }
   const int64_t nrows_all = (int64_t)a.s_total * a.B * a.Hk * a.R;
   for (int b = 0; b < a.B && ck.ok; ++b) {
     for (int kvh = 0; kvh < a.Hk && ck.ok; ++kvh) {
@@ -74,8 +88,19 @@ void check_kernel1(const AttnArgs& a, bool dmask, const AttnExtents& ex, Checker
           kstart = (int64_t)split * a.kps;
           kend = std::min(kstart + a.kps, a.n_pre);
         }
-        const int64_t nkeys = kend - kstart;
-        const int ntiles = nkeys > 0 ? (int)((nkeys + G::KT - 1) / G::KT) : 0;
+        // Causal one-split calls: every row block ends at its own key (the
+        // lengths of a batch are not known here: the longest).  The blocks'
+        // tiles differ in the last one only: all tiles of the longest block
+        // and the last tile of the others are walked.
+        const bool cut = a.direct != 0 && a.causal != 0;
+        const int rpb = attn_rows_per_block();
+        const auto tiles_to = [&](int64_t e) { return e > kstart ? (int)((e - kstart + G::KT - 1) / G::KT) : 0; };
+        if (cut) {
+          int64_t longest = kstart;
+          for (int rb = 0; rb < a.n_rb; ++rb) longest = std::max(longest, causal_kend(rb, rpb, a.M, a.R, a.n_pre - a.M, kend));
+          kend = longest;
+        }
+        const int ntiles = tiles_to(kend);
         const bool paged = src.pt != nullptr;
         int64_t pt_lo = 0;
         if (paged && ntiles > 0) {
@@ -101,7 +126,7 @@ void check_kernel1(const AttnArgs& a, bool dmask, const AttnExtents& ex, Checker
         }
         const int mode = dma_mode<D>(src);
         const int64_t pages[2] = {0, paged ? src.n_phys - 1 : 0};
-        for (int t = 0; t < ntiles && ck.ok; ++t) {
+        const auto check_tile = [&](int t, int64_t kend) {
           const int stage = t & (G::STAGES - 1);
           const int64_t kb = kstart + (int64_t)t * G::KT;
           for (int i = 0; i < 2 * G::NINS && ck.ok; ++i) {
@@ -172,10 +197,23 @@ void check_kernel1(const AttnArgs& a, bool dmask, const AttnExtents& ex, Checker
               ck.range(ex.dmask, elem_addr(a.dmask, b * a.dm_sb + kb * a.dm_sn, 1), 1, "byte-mask read");
             }
           }
-        }
+        };
+        for (int t = 0; t < ntiles && ck.ok; ++t) check_tile(t, kend);
         // Query rows and partial outputs of every row block.
         for (int rb = 0; rb < a.n_rb && ck.ok; ++rb) {
-          const int rpb = attn_rows_per_block();
+          if (cut) {
+            const int64_t e = causal_kend(rb, rpb, a.M, a.R, a.n_pre - a.M, kend);
+            // Every row of the block sees no key from e on.
+            for (int r = rb * rpb; r < std::min(a.R, (rb + 1) * rpb); ++r)
+              ck.cond(std::min(kend, a.n_pre - a.M + 1 + r % a.M) <= e, "causal key end below a row's last key");
+            if (tiles_to(e) > 0) check_tile(tiles_to(e) - 1, e);
+          }
+          if (dmask) {
+            const int waves = mask_waves(rb, rpb / 32, a.R), stride = mask_stride(waves), span = mask_span(stride);
+            ck.cond(waves > 0 && (stride & 1) == 1 && span >= G::STAGES && span % G::STAGES == 0 && span <= stride &&
+                        (waves * 32 - 1) * stride + span <= kMaskWords,
+                    "byte-mask window outside its LDS words");
+          }
           for (int r = rb * rpb; r < std::min(a.R, (rb + 1) * rpb) && ck.ok; ++r) {
             const int g = r / a.M, mi = r - g * a.M;
             const int m = mi;  // row_perm entries are clamped into [0, M) by the kernel
