@@ -11,6 +11,7 @@ attention tests (16-bit probabilities and split results: relative 1e-2).
 import pytest
 import torch
 
+from diffspec_mi355x import _ext
 from diffspec_mi355x.runtime.bundle_verifier import FusedBundleVerifier, PagedBundleVerifier
 
 pytestmark = pytest.mark.gpu
@@ -66,6 +67,9 @@ def test_byte_mask_sizes(gpu, B, M, H, Hk, D, N, kind):
     q, k, v = (torch.randn(s, generator=g, device=gpu).to(torch.float16) for s in
                ((B, M, H, D), (B, N, Hk, D), (B, N, Hk, D)))
     mask = _mask((1, M, N), N + M, gpu, kind)
+    if N == 2597:  # one split of 82 tiles, windows of 76 (20480 words for 256 rows)
+        ws = _ext.load().dsv_attn_workspace_bytes(B, M, H, Hk, D, N, 0, 0)
+        assert ws == B * H * M * (D * 2 + 8), "the plan has more than one split: the window is not refilled"
     got = FusedBundleVerifier(device="cuda").verify_bundle(q, k, v, [mask])
     _check(got, _reference(q, k, v, mask != 0), f"N={N} {kind}")
 

@@ -14,6 +14,7 @@ import math
 import pytest
 import torch
 
+from diffspec_mi355x import _ext
 from diffspec_mi355x.runtime.attention_compat import flash_attn_with_kvcache
 from diffspec_mi355x.runtime.bundle_verifier import FusedBundleVerifier, PagedBundleVerifier
 from diffspec_mi355x.runtime.tree_attention import tree_verify
@@ -27,6 +28,8 @@ B, M, H, N = 16, 3, 16, 160  # B x H = 256 units: one split on 256 CUs or fewer
 
 
 def _inputs(gpu, D, dtype, jump):
+    ws = _ext.load().dsv_attn_workspace_bytes(B, M, H, H, D, N, 0, 0)
+    assert ws == B * H * M * (D * 2 + 8), "the plan has more than one split"
     unit = math.sqrt(D) / math.log2(math.e)  # a score of one log2 unit
     q = torch.zeros((B, M, H, D), device=gpu)
     q[..., 0] = q[..., 1] = 1.0
