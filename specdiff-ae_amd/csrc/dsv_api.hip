@@ -321,9 +321,13 @@ int run(const AttnArgs& a_in, const MergeArgs& m, int dtype, int D, bool dmask, 
   // it is 16-bit with 16-byte aligned rows (2048 x 32 rows over 8192 keys: the
   // partials' merge took 56 of 305 us, 250 without; rows are rounded once, not
   // twice) and skips the keys past a causal block's rows (4096 of 4096: 384 ->
-  // 169 us).
-  a.direct = !dmask && !a.has_tree && a.pre.pt == nullptr && a.pre.fast32 != 0 && dtype != DSV_F32 && a.s_total == 1 && m.weight == nullptr && m.out_dtype != DSV_F32 &&
-             (reinterpret_cast<uintptr_t>(m.out) & 15) == 0 && ((m.o_sb | m.o_sm | m.o_sh) & 7) == 0;
+  // 169 us).  Outputs that overlap an input go through the merge, which starts
+  // when every input has been read.
+  const auto apart = [](const Extent& x, const Extent& y) { return x.hi <= y.lo || y.hi <= x.lo; };
+  const auto outside = [&](const Extent& o) { return apart(o, ex.q) && apart(o, ex.pre_k) && apart(o, ex.pre_v); };
+  a.direct = !dmask && !a.has_tree && a.pre.pt == nullptr && a.pre.fast32 != 0 && dtype != DSV_F32 && a.s_total == 1 &&
+             m.weight == nullptr && m.out_dtype != DSV_F32 && (reinterpret_cast<uintptr_t>(m.out) & 15) == 0 &&
+             ((m.o_sb | m.o_sm | m.o_sh) & 7) == 0 && outside(ex.out) && outside(ex.lse);
   if (a.direct) {
     a.out = static_cast<uint16_t*>(m.out);
     a.direct = m.out_dtype == DSV_F16 ? 2 : 1;

@@ -167,12 +167,12 @@ __global__ void __launch_bounds__(lm_threads(CB), 2) lmhead_stats_kernel(const L
   };
 
   // Step s (W buffer b = s mod NB): the loads of h(s+HD) and W(s+NB-1) issued,
-  // MFMAs on W(s) and h(s) (its B operands read from LDS one sub-step ahead),
-  // h(s+1) into the other LDS buffer, one barrier.  Loads complete in order:
-  // with HD = 2, h(s+1) was issued a step earlier, so the wait for it leaves
-  // W(s+2), h(s+2) and W(s+3) in flight; with HD = 1 it drains all W but the
-  // newest step, which two workgroups per CU hide (64 rows: 3% faster than
-  // HD = 2 and four W buffers).
+  // MFMAs on W(s) and h(s) (its B operands read from LDS ahead of them), h(s+1)
+  // into the other LDS buffer, one barrier.  Loads complete in order: with HD =
+  // 2, h(s+1) was issued a step earlier, so the wait for it leaves W(s+2),
+  // h(s+2) and W(s+3) in flight; with HD = 1 it drains all W but the newest
+  // step, which two workgroups per CU hide (64 rows: 3% faster than HD = 2 and
+  // four W buffers).
   auto step = [&](auto buf_c, int s) {
     constexpr int b = decltype(buf_c)::value;
     const uint8_t* hb = (s & 1) ? hb1 : hb0;

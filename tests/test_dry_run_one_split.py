@@ -55,6 +55,32 @@ def test_one_split_strided_and_unaligned_output(dry, dt, pad, off):
     ok(dry, rc, "flash")
 
 
+def test_outputs_over_inputs_take_the_merge(dry):
+    """The attention kernel's blocks read q, k and v until the last one ends: an output
+    that overlaps them is written by the merge, as one of unaligned rows is (the number
+    of checked accesses tells the two apart)."""
+    B, M, H, D = 16, 40, 16, 64
+    lib = dry
+
+    def checks(out_of, lse_of, off=0):
+        a = Alloc()
+        t = {n: tensor(a, (B, M, H, D)) for n in ("q", "k", "v", "out")}
+        lse = tensor(a, (B, H, M), _ext.DSV_F32)
+        if lse_of:
+            lse.data = t[lse_of].data
+        t[out_of].data += off
+        ws = lib.dsv_attn_workspace_bytes(B, M, H, H, D, M, 0, 0)
+        rc = lib.dsv_flash_attn_with_kvcache(ctypes.byref(t["q"]), ctypes.byref(t["k"]), ctypes.byref(t["v"]), ctypes.byref(none()),
+                                             M, 1, ctypes.byref(t[out_of]), ctypes.byref(lse), a.take(ws), ws, None)
+        ok(lib, rc, f"out over {out_of}, lse over {lse_of}")
+        return lib.dsv_dry_run_checks()
+
+    direct, merged = checks("out", None), checks("out", None, 2)
+    assert direct != merged
+    for out_of, lse_of in (("q", None), ("k", None), ("v", None), ("out", "q"), ("out", "v")):
+        assert checks(out_of, lse_of) == merged, (out_of, lse_of)
+
+
 # Row blocks of 1 to 8 waves, several blocks, more tiles than a window holds.
 @pytest.mark.parametrize("B,M,H,Hk,D,N", [(1, 1, 1, 1, 64, 31), (1, 40, 4, 4, 128, 700), (1, 65, 2, 1, 64, 333), (2, 100, 4, 2, 64, 999),
                                          (1, 150, 1, 1, 128, 400), (1, 180, 1, 1, 64, 100), (1, 200, 1, 1, 64, 129),

@@ -122,3 +122,21 @@ def test_strided_and_unaligned_outputs(gpu, dtype, pad, off, direct):
     rest = buf.clone()
     rest[off:].view(B, M, H, D + pad)[..., :D] = 7.5
     assert (rest == 7.5).all(), "elements between the rows"
+
+
+@pytest.mark.parametrize("over", ["q", "k", "v"])
+def test_output_over_an_input(gpu, over):
+    B, M, H, D = 16, 300, 16, 128
+    print(f"[direct output] out over {over}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(3)
+    t = {n: torch.randn((B, M, H, D), generator=g, device=gpu).to(torch.bfloat16) for n in ("q", "k", "v")}
+    want, want_lse = flash_attn_with_kvcache(t["q"], t["k"], t["v"], causal=True, return_softmax_lse=True)
+    lib, nb = _ext.load(), _ext.load().dsv_attn_workspace_bytes(B, M, H, H, D, M, 0, 0)
+    ws = torch.empty(nb, dtype=torch.uint8, device=gpu)
+    lse = torch.empty_like(want_lse)
+    rc = lib.dsv_flash_attn_with_kvcache(_ext.desc(t["q"]), _ext.desc(t["k"]), _ext.desc(t["v"]), _ext.desc(None), M, 1,
+                                         _ext.desc(t[over]), _ext.desc(lse), ws.data_ptr(), nb, _ext.stream_of(gpu))
+    _ext.check(rc, "flash_attn_with_kvcache")
+    torch.cuda.synchronize()
+    # (bf16 partials of one split, merged, round to the directly written row)
+    assert torch.equal(t[over], want) and torch.equal(lse, want_lse)
