@@ -728,7 +728,7 @@ template <typename LT, int NT, typename F>
 __device__ __forceinline__ void row_sweep_words(const LT* x, int64_t lo, int64_t hi, F&& f);
 template <typename LT>
 constexpr int kRadixWords = sizeof(LT) == 2 ? 32768 : 4 * kCap;  // LDS words of radix_row
-template <typename LT>
+template <typename LT, bool ALL>
 __device__ __forceinline__ void radix_row(const AcceptArgs& a, int64_t row, float m, uint32_t* raw);
 
 // Four waves per SIMD (at most 128 VGPRs): two 512-thread rows share a CU.
@@ -1261,7 +1261,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) sa
   // ---- not decided here ---------------------------------------------------------
   if constexpr (COUNT) {
     __syncthreads();  // the row's LDS above is read no more
-    radix_row<LT>(a, row, m, raw);
+    radix_row<LT, false>(a, row, m, raw);
   } else {  // the radix kernel takes the row (status 2, with m)
     if (tid == 0) a.sel[row] = make_uint4(__float_as_uint(m), 0u, 0u, 2u);
   }
@@ -1316,10 +1316,10 @@ __device__ __forceinline__ T block_excl(T v, T* scratch, T& total) {
 // The digit passes, which form the mass of every entry in double, took 206 us.
 // A counter that overflows shows as a total below V (each overflow loses 65535
 // or 65536); such rows take the digit passes below, as f32 rows do.
-// (m: the row maximum of y; 16-bit logits: not read.  raw: kRadixWords<LT> LDS words.)
+// (m: the row maximum of y; ALL, 16-bit logits: found here.  raw: kRadixWords<LT> LDS words.)
 template <typename LT>
 constexpr int kRadixList = sizeof(LT) == 2 ? kVList : 2 * kCap;  // kept entries drawn here
-template <typename LT>
+template <typename LT, bool ALL>
 __device__ __forceinline__ void radix_row(const AcceptArgs& a, int64_t row, float m, uint32_t* raw) {
   constexpr bool k16 = sizeof(LT) == 2;
   const int t = (int)(row / a.M), i = (int)(row % a.M);
@@ -1390,7 +1390,7 @@ __device__ __forceinline__ void radix_row(const AcceptArgs& a, int64_t row, floa
     // A wave's word of one it is a group: 64 words, which most rows leave empty
     // (a bf16 binade is one group), so that the loops below skip it.
     uint32_t cw[kIt];
-    uint32_t nc = 0, kmax = 0;
+    uint32_t nc = 0;
     const int wtop = kVWords - 1 - tid;
 #pragma unroll
     for (int it = 0; it < kIt; ++it) {
@@ -1406,30 +1406,45 @@ __device__ __forceinline__ void radix_row(const AcceptArgs& a, int64_t row, floa
     static_assert(2 * (kVWords - kRadixThreads) <= (int)kInfKey && 2 * kRadixThreads > (int)kNegInfKey, "first and last words");
     drop(0, 0u, kInfKey);
     drop(kIt - 1, kNegInfKey + 1u, 0xFFFFu);
+    bool whole;  // no counter overflowed (a row whose maximum is known takes one
+                 // reduction in place of four: 2 us a call)
+    if constexpr (!ALL) {
+      nc -= pad;
 #pragma unroll
-    for (int it = kIt - 1; it >= 0; --it)
-      if (cw[it] != 0u) kmax = 2u * (uint32_t)(wtop - kRadixThreads * it) + ((cw[it] >> 16) != 0u ? 1u : 0u);
-    uint32_t total = 0, npad = 0;
-    block_excl<uint32_t, kRadixThreads>(nc, scan_u, total);
-    block_excl<uint32_t, kRadixThreads>(pad, scan_u, npad);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o));
-    __syncthreads();
-    if (lane == 0) scan_u[tid >> 6] = kmax;
-    __syncthreads();
-    for (int w = 0; w < kRadixThreads / 64; ++w) kmax = max(kmax, scan_u[w]);
-    if (total != (uint32_t)V + npad) {
-      // A counter overflowed: the row maximum by a pass, then the digit passes.
-      m = thread_max<LT, kRadixThreads>(x, V);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+      for (int o = 32; o > 0; o >>= 1) nc += (uint32_t)__shfl_xor((int)nc, o);
+      if (lane == 0) scan_u[tid >> 6] = nc;
       __syncthreads();
-      if (lane == 0) scan_u[tid >> 6] = __float_as_uint(m);
-      __syncthreads();
-      for (int w = 0; w < kRadixThreads / 64; ++w) m = fmaxf(m, __uint_as_float(scan_u[w]));
-      if (m > kNegInfF) m = warp_y<LT>(f_to_raw<LT>(m), wp);
+      uint32_t total = 0;
+      for (int w = 0; w < kRadixThreads / 64; ++w) total += scan_u[w];
+      whole = total == (uint32_t)V;
     } else {
-      m = kmax > kNegInfKey ? warp_y<LT>(f_to_raw<LT>(key16_to_f<LT>(kmax)), wp) : kNegInfF;
+      uint32_t kmax = 0;
+#pragma unroll
+      for (int it = kIt - 1; it >= 0; --it)
+        if (cw[it] != 0u) kmax = 2u * (uint32_t)(wtop - kRadixThreads * it) + ((cw[it] >> 16) != 0u ? 1u : 0u);
+      uint32_t total = 0, npad = 0;
+      block_excl<uint32_t, kRadixThreads>(nc, scan_u, total);
+      block_excl<uint32_t, kRadixThreads>(pad, scan_u, npad);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o));
+      __syncthreads();
+      if (lane == 0) scan_u[tid >> 6] = kmax;
+      __syncthreads();
+      for (int w = 0; w < kRadixThreads / 64; ++w) kmax = max(kmax, scan_u[w]);
+      whole = total == (uint32_t)V + npad;
+      if (!whole) {
+        // The row maximum by a pass, then the digit passes.
+        m = thread_max<LT, kRadixThreads>(x, V);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+        __syncthreads();
+        if (lane == 0) scan_u[tid >> 6] = __float_as_uint(m);
+        __syncthreads();
+        for (int w = 0; w < kRadixThreads / 64; ++w) m = fmaxf(m, __uint_as_float(scan_u[w]));
+        if (m > kNegInfF) m = warp_y<LT>(f_to_raw<LT>(m), wp);
+      } else {
+        m = kmax > kNegInfKey ? warp_y<LT>(f_to_raw<LT>(key16_to_f<LT>(kmax)), wp) : kNegInfF;
+      }
     }
     if (!(m > kNegInfF)) {  // no finite logit: nothing is kept (token 0)
       if (tid == 0) finish(0.0, -1);
@@ -1475,7 +1490,7 @@ __device__ __forceinline__ void radix_row(const AcceptArgs& a, int64_t row, floa
       if (tid < kIt * kWv) gtab[tid] = ge;
     }
     __syncthreads();
-    if (total == (uint32_t)V + npad && D <= (uint32_t)kVWords) {  // uniform over the block
+    if (whole && D <= (uint32_t)kVWords) {  // uniform over the block
       // The distinct values in descending order, (key << 16) | count, where
       // the counters were (every thread holds its own in registers).
       uint32_t* const vals = raw;
@@ -1815,17 +1830,18 @@ __device__ __forceinline__ void radix_row(const AcceptArgs& a, int64_t row, floa
   if (tid == 0) a.sel[row] = make_uint4(tk, ystar, istar, 0u);
 }
 
-template <typename LT>
-__global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const AcceptArgs a, int all) {
+template <typename LT, bool ALL>
+__global__ void __launch_bounds__(kRadixThreads) sample_radix_kernel(const AcceptArgs a) {
+  static_assert(!ALL || sizeof(LT) == 2, "only the value counts find the row maximum");
   __shared__ __align__(16) uint32_t raw[kRadixWords<LT>];
   const int64_t row = blockIdx.x;
   float m = 0.f;
-  if (sizeof(LT) != 2 || all == 0) {
+  if constexpr (!ALL) {
     const uint4 st = a.sel[row];
     if (st.w != 2u) return;
     m = __uint_as_float(st.x);
   }
-  radix_row<LT>(a, row, m, raw);
+  radix_row<LT, ALL>(a, row, m, raw);
 }
 
 // Gumbel-max draw over one vocabulary range of one row.
@@ -2295,8 +2311,8 @@ hipError_t launch_sample_t(const AcceptArgs& a, hipStream_t s) {
   // 16-bit rows of one round of the CUs: the regions' head, else the value counts,
   // in one kernel.  (Microseconds of a call on rows that are all sure of their
   // token / of which a tenth share the mass between thousands; 64 rows, top-p 0.9.
-  // 128256 entries: 46 / 76, counts alone 52 / 72, heads and histograms first 49 /
-  // 360; 32000: 27 / 46, 38 / 43, 31 / 162.)
+  // 128256 entries: 46 / 74, counts alone 52 / 72, heads and histograms first 49 /
+  // 360; 32000: 27 / 45, 38 / 43, 31 / 162.)
   // Straight to the counts (all) where the row maximum that comes before a head
   // costs more than a head saves: top-k alone from 65536 entries (64 rows: 53 on
   // sure rows, 58 with heads tried first, 128 with heads and histograms; 512 rows
@@ -2312,7 +2328,7 @@ hipError_t launch_sample_t(const AcceptArgs& a, hipStream_t s) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   } else if (a.sel != nullptr && all) {
-    hipLaunchKernelGGL(sample_radix_kernel<LT>, dim3(rows), dim3(kRadixThreads), 0, s, a, 1);
+    if constexpr (sizeof(LT) == 2) hipLaunchKernelGGL((sample_radix_kernel<LT, true>), dim3(rows), dim3(kRadixThreads), 0, s, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   } else if (a.sel != nullptr) {
@@ -2324,7 +2340,7 @@ hipError_t launch_sample_t(const AcceptArgs& a, hipStream_t s) {
       hipLaunchKernelGGL((sample_select_kernel<LT, 1024>), dim3(rows), dim3(1024), 0, s, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(sample_radix_kernel<LT>, dim3(rows), dim3(kRadixThreads), 0, s, a, 0);
+    hipLaunchKernelGGL((sample_radix_kernel<LT, false>), dim3(rows), dim3(kRadixThreads), 0, s, a);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
