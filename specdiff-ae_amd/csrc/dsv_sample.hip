@@ -2318,7 +2318,7 @@ hipError_t launch_sample_t(const AcceptArgs& a, hipStream_t s) {
   // sure rows, 58 with heads tried first, 128 with heads and histograms; 512 rows
   // 98 and 218), and bf16 rows of that length that fill three quarters of the CUs,
   // whose passes are bound by memory (256 rows: 55 / 74, 52 / 82, 56 / 376; f16 rows
-  // count slower: 65 / 86, 57 / 94, 61 / 486).  More rows than CUs would take a round
+  // count slower: 65 / 86, 56 / 92, 61 / 486).  More rows than CUs would take a round
   // each in the counts: 512 rows, none open, 100 against 83.
   const int64_t ncu = a.cus > 0 ? a.cus : 256;
   const bool k16 = sizeof(LT) == 2, fits = (int64_t)rows <= ncu, full = 4 * (int64_t)rows >= 3 * ncu;
